@@ -16,6 +16,8 @@ QUANT_IN = {"fp16": 0, "bf16": 1, "fp32": 2}
 QUANT_OUT = {"fp8": 0, "int8": 1}
 QUANT_MODE = {"recip_trunc": 0, "div_trunc": 1, "div_nearest": 2}
 
+MOE_SORT_MAX_EXPERTS = 512
+
 # (name, restype, argtypes) for every symbol include/flygemm.h declares
 _P = ctypes.c_void_p
 _I = ctypes.c_int32
@@ -35,6 +37,8 @@ SIGNATURES = [
      [_P, _P, _P, _F, _F, _P, _P, _F, _P] + [_I] * 12 + [_P, _I, _P]),
     ("flygemm_moe_blockscale_gemm1", ctypes.c_int, [_P, _P, _P, _F, _F, _P, _P, _F, _P] + [_I] * 11 + [_P]),
     ("flygemm_moe_blockscale_gemm2", ctypes.c_int, [_P, _P, _P, _F, _F, _P, _P, _F, _P] + [_I] * 12 + [_P]),
+    ("flygemm_moe_sort_scratch", ctypes.c_int32, [_I] * 3),
+    ("flygemm_moe_sort", ctypes.c_int, [_P] * 8 + [_I] * 5 + [_P]),
     ("flygemm_num_variants", ctypes.c_int32, []),
     ("flygemm_variant_name", ctypes.c_char_p, [_I]),
     ("flygemm_select_variant", ctypes.c_int32, [_I, _I, _I, _I, _I]),

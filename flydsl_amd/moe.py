@@ -20,6 +20,45 @@ from __future__ import annotations
 
 import torch
 
+from . import _lib
+
+
+def _plain_cuda(*ts) -> bool:
+    """Tensors whose values a kernel may read and write by pointer in place of torch's own
+    operators: ordinary tensors of one GPU, outside autograd, functorch, tracing and dispatch modes."""
+    dev = ts[0].device
+    if dev.type != "cuda" or any(type(t) is not torch.Tensor or t.device != dev for t in ts):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+        return False
+    C = torch._C
+    return not (C._len_torch_dispatch_stack() or C._len_torch_function_stack() or torch.compiler.is_compiling()
+                or C._get_tracing_state() is not None or C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
+def _sort_kernel(topk_ids, topk_weights, E, bs, expert_mask):
+    """moe_sorting through flygemm_moe_sort (one or two launches, no synchronisation)."""
+    dev = topk_ids.device
+    M, topk = topk_ids.shape
+    max_pad = M * topk + E * bs - topk
+    ids = topk_ids if topk_ids.dtype in (torch.int32, torch.int64) else topk_ids.to(torch.int64)
+    ids, w = ids.contiguous(), topk_weights.to(torch.float32).contiguous()
+    mask = None if expert_mask is None else (expert_mask.reshape(-1)[:E].to(torch.int64) != 0).contiguous()
+    sorted_ids = torch.empty(max_pad, dtype=torch.int32, device=dev)
+    sorted_w = torch.empty(max_pad, dtype=torch.float32, device=dev)
+    sorted_eids = torch.empty((max_pad + bs - 1) // bs, dtype=torch.int32, device=dev)
+    post = torch.empty(2, dtype=torch.int32, device=dev)
+    lib = _lib.load()
+    n = lib.flygemm_moe_sort_scratch(M, topk, E)
+    scratch = torch.empty(n, dtype=torch.int32, device=dev) if n else None
+    rc = lib.flygemm_moe_sort(sorted_ids.data_ptr(), sorted_w.data_ptr(), sorted_eids.data_ptr(), post.data_ptr(),
+                              scratch.data_ptr() if n else None, ids.data_ptr(), w.data_ptr(),
+                              None if mask is None else mask.data_ptr(), M, topk, E, bs,
+                              int(ids.dtype == torch.int64), torch.cuda.current_stream(dev).cuda_stream)
+    _lib.check(rc, "flygemm_moe_sort")
+    return sorted_ids, sorted_w, sorted_eids, post
+
 
 def moe_sorting(topk_ids: torch.Tensor, topk_weights: torch.Tensor, num_experts: int, block_size: int,
                 expert_mask: torch.Tensor | None = None):
@@ -32,6 +71,18 @@ def moe_sorting(topk_ids: torch.Tensor, topk_weights: torch.Tensor, num_experts:
     dev = topk_ids.device
     M, topk = topk_ids.shape
     max_pad = M * topk + E * bs - topk
+    # On the GPU: the counting-sort kernel (csrc/moe_sort.hip) in place of about 40 operators, two
+    # of which (bincount, torch.tensor) wait for the device.  Measured on MI355X, back to back: 8
+    # tokens, 256 experts, top-8 16.5 us against 398; 8192 tokens, 128 experts, top-8 20.0 against 439.
+    # More experts than the kernel's counters, a top-k above the experts (whose rows may not fit
+    # the buffers), empty routings and masks shorter than the experts take the operators below.
+    if (0 < topk <= E <= _lib.MOE_SORT_MAX_EXPERTS and M > 0 and max_pad < 2**31 - 2**16
+            and (expert_mask is None or expert_mask.numel() >= E)
+            and _plain_cuda(*(t for t in (topk_ids, topk_weights, expert_mask) if t is not None))):
+        if dev.index == torch.cuda.current_device():
+            return _sort_kernel(topk_ids, topk_weights, E, bs, expert_mask)
+        with torch.cuda.device(dev):
+            return _sort_kernel(topk_ids, topk_weights, E, bs, expert_mask)
     max_blocks = (max_pad + bs - 1) // bs
 
     flat = topk_ids.reshape(-1).to(torch.int64)

@@ -245,6 +245,21 @@ int flygemm_moe_gemm2_reduce_noalloc(void* out, const void* a2, const void* w, c
                                      int32_t doweight_stage2, int32_t group_size, const void* valid_mask,
                                      int32_t zero_intermediate, void* stream);
 
+/* Routing metadata of the MoE GEMMs from a router's choice: topk_ids [tokens][topk] (int32, or
+ * int64 with ids_64bit != 0) and topk_weights fp32 [tokens][topk], as the reference harness's
+ * moe_sorting_torch_native gives it (tests/kernels/test_moe_gemm.py:97-160): sorted_ids int32 and
+ * sorted_weights fp32 [tokens*topk + experts*block - topk], sorted_expert_ids int32 [that / block,
+ * rounded up], num_post_pad int32 [2].  Ids outside [0, experts), and those of experts with
+ * expert_mask[e] == 0 (bytes, [experts]; NULL: none), are dropped, and the experts that the mask
+ * keeps are renumbered.  experts at most FLYGEMM_MOE_SORT_MAX_EXPERTS, topk at most experts.
+ * scratch: int32 [flygemm_moe_sort_scratch(tokens, topk, experts)] (no scratch where that is 0).
+ * One launch for up to 8192 routes, two above; nothing is synchronized. */
+#define FLYGEMM_MOE_SORT_MAX_EXPERTS 512
+int32_t flygemm_moe_sort_scratch(int32_t tokens, int32_t topk, int32_t experts);
+int flygemm_moe_sort(int32_t* sorted_ids, float* sorted_weights, int32_t* sorted_expert_ids, int32_t* num_post_pad,
+                     int32_t* scratch, const void* topk_ids, const float* topk_weights, const uint8_t* expert_mask,
+                     int32_t tokens, int32_t topk, int32_t experts, int32_t block, int32_t ids_64bit, void* stream);
+
 /* Kernel variant table (replaces the reference's per-call tile kwargs,
  * kernels/preshuffle_gemm.py:39-53, with a static table). */
 int32_t flygemm_num_variants(void);
