@@ -680,14 +680,16 @@ __global__ void __launch_bounds__(WM * WN * 64) moe_gemm_kernel(MoeArgs p) {
 }
 
 // Reduce mode, second kernel: y[t][d] = sum over slots k of x[t][k][d] (slots with
-// valid_mask[t][k] == 0 skipped when a mask is given), fp32 sums, one 16-byte vector of d per
-// thread; x is read once, so it is loaded non-temporally (reference compile_moe_reduction,
-// kernels/moe_gemm_2stage.py:2484-2604).  DT: 0 fp16, 1 bf16, 2 fp32.
+// mask[t][k] == 0 skipped when a mask is given), fp32 sums in slot order, one 16-byte vector of d
+// per thread; x is read once, so it is loaded non-temporally (reference compile_moe_reduction,
+// kernels/moe_gemm_2stage.py:2484-2604).  DT: 0 fp16, 1 bf16, 2 fp32.  Bound by reading x.  Up to eight slots' loads are in flight at once (one load at a time
+// left each thread waiting out the memory latency per slot); a masked slot is not read.
 template <int DT>
 __global__ void __launch_bounds__(256) moe_reduce_kernel(void* y, const void* x, const int8_t* mask, int tokens,
                                                          int topk, int D) {
   constexpr int ESZ = DT == 2 ? 4 : 2;
   constexpr int VE = 16 / ESZ;                 // elements per vector
+  constexpr int U = 8;                         // slots in flight
   const int vpr = D / VE;                      // vectors per row
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (long)tokens * vpr) return;
@@ -709,19 +711,17 @@ __global__ void __launch_bounds__(256) moe_reduce_kernel(void* y, const void* x,
       for (int q = 0; q < 8; ++q) acc[q] += (float)h[q];
     }
   };
-  if (topk == 8 && !mask) {
-    // the common case: all eight slots' loads in flight at once, then the sums in slot order
-    // (one load at a time left each thread waiting out the memory latency per slot)
-    i32x4 w[8];
+  for (int k0 = 0; k0 < topk; k0 += U) {
+    i32x4 w[U];
+    bool use[U];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) w[k] = __builtin_nontemporal_load(src + (long)k * vpr);
+    for (int k = 0; k < U; ++k) use[k] = k0 + k < topk && (!mask || mask[(long)t * topk + k0 + k] != 0);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) add(w[k]);
-  } else {
-    for (int k = 0; k < topk; ++k) {
-      if (mask && mask[(long)t * topk + k] == 0) continue;
-      add(__builtin_nontemporal_load(src + (long)k * vpr));
-    }
+    for (int k = 0; k < U; ++k)
+      if (use[k]) w[k] = __builtin_nontemporal_load(src + (long)(k0 + k) * vpr);
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      if (use[k]) add(w[k]);
   }
   i32x4* dst = (i32x4*)y + idx;
   if constexpr (DT == 2) {

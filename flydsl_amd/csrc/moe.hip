@@ -463,9 +463,66 @@ int noalloc_scratch(void** out, const char* what, hipStream_t stream) {
   return 0;
 }
 
+// y [tokens][D] = the reduction of x [tokens][topk][D] (checked arguments)
+int reduce_launch(void* y, const void* x, const void* mask, int tokens, int topk, int D, int dtype, hipStream_t stream) {
+  const long n = (long)tokens * (D / (dtype == FLYGEMM_OUT_F32 ? 4 : 8));
+  const long g = (n + 255) / 256;
+  if (g >= (1L << 31)) return fail(hipErrorInvalidValue, "moe_reduce: too large");
+  void (*fn)(void*, const void*, const int8_t*, int, int, int) =
+      dtype == FLYGEMM_OUT_FP16 ? moe_reduce_kernel<0> : dtype == FLYGEMM_OUT_BF16 ? moe_reduce_kernel<1>
+                                                                                   : moe_reduce_kernel<2>;
+  hipLaunchKernelGGL(fn, dim3((unsigned)g), dim3(256), 0, stream, y, x, (const int8_t*)mask, tokens, topk, D);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(e, "launch of moe_reduce failed: %s", hipGetErrorString(e));
+  return 0;
+}
+
 // Zero fill in place of hipMemsetAsync, so the call can be captured in a graph.
 __global__ void __launch_bounds__(256) zero_fill_kernel(uint4* p, long n) {
   for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) p[i] = uint4{0, 0, 0, 0};
+}
+
+int zero_fill(void* p, long bytes, const char* what, hipStream_t s) {
+  const long n = bytes / 16;
+  const long g = (n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048;
+  hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)g), dim3(256), 0, s, (uint4*)p, n);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(e, "%s: launch of the zero fill failed: %s", what, hipGetErrorString(e));
+  return 0;
+}
+
+// mask[t*topk + s] = 1 for every route that a stage-2 call on this metadata writes a row of (the
+// entries that the GEMM kernels take); the mask was zeroed before.
+__global__ void __launch_bounds__(256) route_mask_kernel(int8_t* mask, const int32_t* sorted_ids,
+                                                         const int32_t* expert_ids, const int32_t* num_valid,
+                                                         int tokens, int topk, int blocks, int experts, int tile_m) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  const long b = i / tile_m;
+  const int nbv = min((num_valid[0] + tile_m - 1) / tile_m, blocks);
+  if (b >= nbv) return;
+  const int e = expert_ids[b];
+  if (e < 0 || e >= experts) return;
+  const int id = sorted_ids[i];
+  const int t = id & 0xFFFFFF, s = (int)((uint32_t)id >> 24);
+  if (t < tokens && s < topk) mask[(long)t * topk + s] = 1;
+}
+
+// Rows bytes from which flygemm_moe_gemm2_reduce marks the routes that have a row (a byte each,
+// read by the reduction) in place of zeroing the rows: two small launches against a pass of
+// writes.  Graph-timed on MI355X, DS-TP8 dims, zeroed rows against the mask: 100 tokens (11 MB)
+// 48.3 us against 47.6, 512 tokens (59 MB) 75.6 against 68.2, 2048 tokens 206.8 against 173.2,
+// 8192 tokens (940 MB) 654 against 468; the second launch costs the host 3 us.
+constexpr long kRouteMaskFrom = 16L << 20;
+
+// Scratch of a reduce-mode stage 2: the per-route rows, then the route mask (0 bytes: none).
+struct ReduceScratch {
+  long rows, mask;
+};
+ReduceScratch reduce_scratch(int tokens, int topk, int model_dim, bool need_zero) {
+  const long routes = (long)tokens * topk;
+  ReduceScratch r{(routes * model_dim * 2 + 255) / 256 * 256, 0};
+  if (need_zero && r.rows >= kRouteMaskFrom) r.mask = (routes + 255) / 256 * 256;
+  return r;
 }
 
 }  // namespace
@@ -536,17 +593,7 @@ int flygemm_moe_reduce(void* y, const void* x, const void* valid_mask, int32_t t
   if (tokens == 0) return 0;
   if (!y || !x) return fail(hipErrorInvalidValue, "moe_reduce: null tensor pointer");
   if (((uintptr_t)y | (uintptr_t)x) & 15) return fail(hipErrorInvalidValue, "moe_reduce: misaligned pointer");
-  const long n = (long)tokens * (model_dim / ve);
-  const long g = (n + 255) / 256;
-  if (g >= (1L << 31)) return fail(hipErrorInvalidValue, "moe_reduce: too large");
-  void (*fn)(void*, const void*, const int8_t*, int, int, int) =
-      dtype == FLYGEMM_OUT_FP16 ? moe_reduce_kernel<0> : dtype == FLYGEMM_OUT_BF16 ? moe_reduce_kernel<1>
-                                                                                   : moe_reduce_kernel<2>;
-  hipLaunchKernelGGL(fn, dim3((unsigned)g), dim3(256), 0, (hipStream_t)stream, y, x, (const int8_t*)valid_mask,
-                     tokens, topk, model_dim);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(e, "launch of moe_reduce failed: %s", hipGetErrorString(e));
-  return 0;
+  return reduce_launch(y, x, valid_mask, tokens, topk, model_dim, dtype, (hipStream_t)stream);
 }
 
 int flygemm_moe_select_tile(int32_t stage, int32_t tokens, int32_t n, int32_t k, int32_t experts, int32_t topk,
@@ -609,15 +656,62 @@ int flygemm_moe_gemm2_reduce_noalloc(void* out, const void* a2, const void* w, c
   void* inter = nullptr;
   if (int rc = noalloc_scratch(&inter, what, s)) return rc;
   pl.args.out = inter;
-  if (zero_intermediate && !valid_mask) {
-    const long n = need / 16;
-    const long g = (n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048;
-    hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)g), dim3(256), 0, s, (uint4*)inter, n);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(e, "%s: launch of the zero fill failed: %s", what, hipGetErrorString(e));
-  }
+  if (zero_intermediate && !valid_mask)
+    if (int rc = zero_fill(inter, need, what, s)) return rc;
   if (int rc = moe_run(pl, what, s)) return rc;
   return flygemm_moe_reduce(out, inter, valid_mask, tokens, topk, model_dim, out_dtype, stream);
+}
+
+int64_t flygemm_moe_gemm2_reduce_scratch(int32_t tokens, int32_t topk, int32_t model_dim, int32_t zero_rows) {
+  if (tokens <= 0 || topk <= 0 || model_dim <= 0) return 0;
+  const ReduceScratch r = reduce_scratch(tokens, topk, model_dim, zero_rows != 0);
+  return r.rows + r.mask;
+}
+
+int flygemm_moe_gemm2_reduce(void* out, void* scratch, int64_t scratch_bytes, const void* a2, const void* w,
+                             const float* scale_a2, const float* scale_w, const int32_t* sorted_token_ids,
+                             const int32_t* sorted_expert_ids, const float* sorted_weights,
+                             const int32_t* num_valid_ids, int32_t tokens, int32_t model_dim, int32_t inter_dim,
+                             int32_t size_expert_ids, int32_t experts, int32_t topk, int32_t tile_m, int32_t tile_n,
+                             int32_t in_dtype, int32_t out_dtype, int32_t doweight_stage2, int32_t blockscale,
+                             int32_t group_size, const void* valid_mask, int32_t zero_rows, void* stream) {
+  const char* what = "moe_gemm2_reduce";
+  if (out_dtype != FLYGEMM_OUT_FP16 && out_dtype != FLYGEMM_OUT_BF16)
+    return fail(hipErrorInvalidValue, "%s: out_dtype %d not supported (fp16 or bf16)", what, out_dtype);
+  if (model_dim > 0 && model_dim % 8 != 0)
+    return fail(hipErrorInvalidValue, "%s: model_dim=%d must be a multiple of 8", what, model_dim);
+  // every check comes before the first launch: a rejected call queues nothing on the stream
+  MoePlan pl;
+  if (int rc = moe_plan(2, scratch, a2, w, scale_a2, scale_w, sorted_token_ids, sorted_expert_ids, sorted_weights,
+                        num_valid_ids, tokens, model_dim, inter_dim, size_expert_ids, experts, topk, tile_m, tile_n,
+                        in_dtype, out_dtype, doweight_stage2, 0, blockscale != 0, group_size, &pl))
+    return rc;
+  if (tokens == 0) return 0;
+  if (!out || !scratch) return fail(hipErrorInvalidValue, "%s: null output or scratch pointer", what);
+  if (((uintptr_t)out | (uintptr_t)scratch) & 15)
+    return fail(hipErrorInvalidValue, "%s: misaligned output or scratch (16 bytes needed)", what);
+  const bool need_zero = zero_rows && !valid_mask;
+  const ReduceScratch r = reduce_scratch(tokens, topk, model_dim, need_zero);
+  if (scratch_bytes < r.rows + r.mask)
+    return fail(hipErrorInvalidValue, "%s: scratch of %ld bytes, needs %ld", what, (long)scratch_bytes, r.rows + r.mask);
+  hipStream_t s = (hipStream_t)stream;
+  const void* mask = valid_mask;
+  if (r.mask) {
+    int8_t* m = (int8_t*)scratch + r.rows;
+    if (int rc = zero_fill(m, r.mask, what, s)) return rc;
+    if (pl.kernel.fn) {
+      const long n = (long)size_expert_ids * tile_m;
+      hipLaunchKernelGGL(route_mask_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, m, sorted_token_ids,
+                         sorted_expert_ids, num_valid_ids, tokens, topk, size_expert_ids, experts, tile_m);
+      hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return fail(e, "%s: launch of the route mask failed: %s", what, hipGetErrorString(e));
+    }
+    mask = m;
+  } else if (need_zero) {
+    if (int rc = zero_fill(scratch, r.rows, what, s)) return rc;
+  }
+  if (int rc = moe_run(pl, what, s)) return rc;
+  return reduce_launch(out, scratch, mask, tokens, topk, model_dim, out_dtype, s);
 }
 
 }  // extern "C"

@@ -82,10 +82,10 @@ class _MoeStage:
         self.blockscale = bool(blockscale)   # fp8 with 1x128 / 128x128 block scales
         self.group_size = int(group_size) if int(group_size) > 0 else -1
 
-    def __call__(self, arg_out, arg_x, arg_w, arg_scale_x, arg_scale_w, arg_sorted_token_ids, arg_expert_ids,
-                 arg_sorted_weights, arg_num_valid_ids, tokens, n_in, k_in, size_expert_ids, stream=None):
+    def _check_args(self, arg_x, arg_w, arg_scale_x, arg_scale_w, arg_sorted_token_ids, arg_expert_ids,
+                    arg_sorted_weights, arg_num_valid_ids, tokens, n_in, k_in, size_expert_ids):
+        """Every check but the output's: the sizes as ints and the data pointers, in the C order."""
         tokens, N, K, blocks = int(tokens), int(n_in), int(k_in), int(size_expert_ids)
-        h_stream = stream_handle(stream)
         if tokens < 0 or blocks < 0:
             raise ValueError(f"invalid tokens={tokens} / size_expert_ids={blocks}")
         want_n, want_k = (self.inter_dim, self.model_dim) if self.stage == 1 else (self.model_dim, self.inter_dim)
@@ -101,9 +101,6 @@ class _MoeStage:
         a_rows = tokens * topk if per_route else tokens
         w_rows = E * 2 * N if self.stage == 1 else E * N
         w_bytes = w_rows * K // 2 if self.in_dtype in _W4 else w_rows * K
-        out_name, out_t = _OUT[self.out_dtype]
-        out_elems = tokens * topk * N if (self.stage == 1 or not self.accumulate) else tokens * N
-        o = device_ptr(arg_out, "arg_out", out_elems, dtypes=(out_t,))
         if self.in_dtype in _T16:
             x = device_ptr(arg_x, "arg_x", a_rows * K, dtypes=(_T16[self.in_dtype],))
             sx = 0  # unscaled activations; the reference passes empty tensors
@@ -128,10 +125,19 @@ class _MoeStage:
         sws = (device_ptr(arg_sorted_weights, "arg_sorted_weights", n_sorted, dtypes=(torch.float32,))
                if self.doweight else 0)
         nv = device_ptr(arg_num_valid_ids, "arg_num_valid_ids", 1, dtypes=(torch.int32,))
+        return (x, w, sx, sw, ids, eids, sws, nv), (tokens, N, K, blocks, E, topk, self.tile_m, self.tile_n)
+
+    def __call__(self, arg_out, arg_x, arg_w, arg_scale_x, arg_scale_w, arg_sorted_token_ids, arg_expert_ids,
+                 arg_sorted_weights, arg_num_valid_ids, tokens, n_in, k_in, size_expert_ids, stream=None):
+        h_stream = stream_handle(stream)
+        ptrs, sizes = self._check_args(arg_x, arg_w, arg_scale_x, arg_scale_w, arg_sorted_token_ids, arg_expert_ids,
+                                       arg_sorted_weights, arg_num_valid_ids, tokens, n_in, k_in, size_expert_ids)
+        out_name, out_t = _OUT[self.out_dtype]
+        rows = sizes[0] * (self.topk if self.stage == 1 or not self.accumulate else 1)
+        o = device_ptr(arg_out, "arg_out", rows * sizes[1], dtypes=(out_t,))
         lib = _lib.load()
         dt = 128 if self.blockscale else _lib.FLYGEMM_IN[self.in_dtype]   # scale_block_k / in_dtype
-        args = (o, x, w, sx, sw, ids, eids, sws, nv, tokens, N, K, blocks, E, topk, self.tile_m, self.tile_n, dt,
-                _lib.FLYGEMM_OUT[out_name], int(self.doweight))
+        args = (o, *ptrs, *sizes, dt, _lib.FLYGEMM_OUT[out_name], int(self.doweight))
         name = f"flygemm_moe_{'blockscale_' if self.blockscale else ''}gemm{self.stage}"
         fn = getattr(lib, name)
         tail = () if self.blockscale else (self.group_size,)
@@ -212,10 +218,11 @@ class MoeGemm2Mode:
 
 class _MoeGemm2ReduceWrapper:
     """Stage 2 in reduce mode (reference ``moe_gemm_2stage.py:2689-2774``): the GEMM writes
-    every route's row of an intermediate [tokens*topk, model_dim] with plain stores, then the
-    reduction sums the top-k rows of each token into ``arg_out``.  The intermediate comes from
-    torch's caching allocator (zeroed unless a valid mask says which rows to read, or
-    ``zero_intermediate=False`` promises every route is written)."""
+    every route's row of an intermediate with plain stores, then the reduction sums the top-k rows
+    of each token into ``arg_out``; one call to the library (``flygemm_moe_gemm2_reduce``).  The
+    intermediate comes from torch's caching allocator.  A route without a row adds nothing: a valid
+    mask says which rows to read, or ``zero_intermediate=False`` promises that every route is
+    written, or else the library finds them itself."""
 
     def __init__(self, gemm2_exe, reduce_exe, topk, model_dim, out_dtype_str="f16", use_mask=False,
                  zero_intermediate=True):
@@ -228,19 +235,32 @@ class _MoeGemm2ReduceWrapper:
     def __call__(self, arg_out, arg_x, arg_w, arg_scale_x, arg_scale_w, arg_sorted_token_ids, arg_expert_ids,
                  arg_sorted_weights, arg_num_valid_ids, tokens_in, n_in, k_in, size_expert_ids_in, valid_mask=None,
                  stream=None):
-        tokens = int(tokens_in)
+        g = self._gemm2_exe
         if stream is None:
             stream = torch.cuda.current_stream()
-        inter = torch.empty(tokens * self._topk, self._model_dim, device=arg_out.device,
-                            dtype=_RED_DT[self._out_dtype_str])
-        if self._zero_intermediate and not self._use_mask:
-            inter.zero_()
-        self._gemm2_exe(inter.view(-1), arg_x, arg_w, arg_scale_x, arg_scale_w, arg_sorted_token_ids, arg_expert_ids,
-                        arg_sorted_weights, arg_num_valid_ids, tokens, n_in, k_in, size_expert_ids_in, stream)
+        h_stream = stream_handle(stream)
+        ptrs, sizes = g._check_args(arg_x, arg_w, arg_scale_x, arg_scale_w, arg_sorted_token_ids, arg_expert_ids,
+                                    arg_sorted_weights, arg_num_valid_ids, tokens_in, n_in, k_in, size_expert_ids_in)
+        tokens = sizes[0]
         if self._use_mask and valid_mask is None:
             raise ValueError("this reduce-mode stage 2 was compiled with a valid mask; pass valid_mask")
+        y = device_ptr(arg_out.view(-1), "Y", tokens * self._model_dim, dtypes=(_RED_DT[self._out_dtype_str],))
         mask = valid_mask.contiguous().view(-1) if self._use_mask else None
-        self._reduce_exe(inter.view(-1), arg_out.view(-1), mask, tokens, stream)
+        mk = device_ptr(mask, "valid_mask", tokens * self._topk, elem_bytes=1) if self._use_mask else 0
+        lib = _lib.load()
+        kinds = (_lib.FLYGEMM_IN[g.in_dtype], _lib.FLYGEMM_OUT[_OUT[g.out_dtype][0]])
+        zero = int(self._zero_intermediate and not self._use_mask)
+        nbytes = lib.flygemm_moe_gemm2_reduce_scratch(tokens, self._topk, self._model_dim, zero)
+        rows = torch.empty(nbytes, dtype=torch.uint8, device=arg_out.device)
+        rc = lib.flygemm_moe_gemm2_reduce(y, rows.data_ptr(), nbytes, *ptrs, *sizes, *kinds, int(g.doweight),
+                                          int(g.blockscale), g.group_size, mk, zero, h_stream)
+        _lib.check(rc, "flygemm_moe_gemm2_reduce")
+        if h_stream != torch.cuda.current_stream(arg_out.device).cuda_stream:
+            # the allocator hands memory out again in the order of the stream it came from
+            other = stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.ExternalStream(h_stream, arg_out.device)
+            rows.record_stream(other)
+            if mask is not None:
+                mask.record_stream(other)
 
     @property
     def mode(self) -> str:

@@ -224,6 +224,21 @@ int flygemm_moe_select_tile(int32_t stage, int32_t tokens, int32_t n, int32_t k,
 int flygemm_moe_reduce(void* y, const void* x, const void* valid_mask, int32_t tokens, int32_t topk,
                        int32_t model_dim, int32_t dtype, void* stream);
 
+/* Stage 2 in reduce mode in one call (reference kernels/moe_gemm_2stage.py:2689-2774): the GEMM
+ * without accumulation into per-route rows, then the reduction of each token's rows into out
+ * [tokens][model_dim] (fp16 or bf16), as flygemm_moe_gemm2 / flygemm_moe_blockscale_gemm2
+ * (blockscale != 0) with accumulate = 0 and flygemm_moe_reduce give it.  With zero_rows != 0 and no
+ * valid_mask, routes that the metadata holds no entry for add nothing.  scratch: 16-byte aligned,
+ * flygemm_moe_gemm2_reduce_scratch(...) bytes (zero_rows 0 there when a valid_mask is given). */
+int64_t flygemm_moe_gemm2_reduce_scratch(int32_t tokens, int32_t topk, int32_t model_dim, int32_t zero_rows);
+int flygemm_moe_gemm2_reduce(void* out, void* scratch, int64_t scratch_bytes, const void* a2, const void* w,
+                             const float* scale_a2, const float* scale_w, const int32_t* sorted_token_ids,
+                             const int32_t* sorted_expert_ids, const float* sorted_weights,
+                             const int32_t* num_valid_ids, int32_t tokens, int32_t model_dim, int32_t inter_dim,
+                             int32_t size_expert_ids, int32_t experts, int32_t topk, int32_t tile_m, int32_t tile_n,
+                             int32_t in_dtype, int32_t out_dtype, int32_t doweight_stage2, int32_t blockscale,
+                             int32_t group_size, const void* valid_mask, int32_t zero_rows, void* stream);
+
 /* Stage 2 in reduce mode in one call that allocates nothing: flygemm_moe_gemm2 with
  * accumulate = 0 into per-route rows [tokens*topk][model_dim] (fp16 or bf16), zeroed first when
  * zero_intermediate != 0 and valid_mask is NULL, then flygemm_moe_reduce of those rows into out

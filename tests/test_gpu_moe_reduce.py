@@ -1,0 +1,75 @@
+"""Reduce-mode stage 2 in one library call against its two steps on rows zeroed first (per-route GEMM,
+then the reduction; both are checked against the oracle in tests/test_gpu_moe.py): equal bit for bit,
+with routes that no expert takes, whether the rows are zeroed or the routes marked."""
+import pytest
+import torch
+
+from flydsl_amd import workloads
+from flydsl_amd.kernels.moe_gemm_2stage import (MoeGemm2Mode, compile_moe_gemm2, compile_moe_gemm2_ex,
+                                                compile_moe_reduction)
+from flydsl_amd.moe import moe_sorting
+
+pytestmark = pytest.mark.gpu
+_DT = {"f16": torch.float16, "bf16": torch.bfloat16}
+
+
+def _problem(tokens, topk, dim, inter, experts, tile_m, kept, gpu):
+    p = workloads.moe_problem(workloads.moe_custom(tokens, dim, inter, experts, topk, tile_m, 64, 128, seed=tokens), gpu)
+    mask = torch.zeros(experts, dtype=torch.int32, device=gpu)
+    mask[:kept] = 1
+    ids, w, eids, post = moe_sorting(p["topk_ids"], p["topk_weights"], experts, tile_m, mask)
+    return p, (ids, eids, w, post[:1].contiguous()), eids.numel()
+
+
+def _args(p, meta, tokens, dim, inter, blocks):
+    return (p["a2"].view(-1), p["w2_shuf"].view(-1), p["sa2"], p["sw2"], *meta, tokens, dim, inter, blocks)
+
+
+# tokens, topk, model_dim, tile_m: rows below and above the 16 MB from which routes are marked; one,
+# two and three groups of eight slots
+CASES = [(40, 8, 1024, 16), (1023, 8, 1024, 32), (1025, 8, 1024, 32), (600, 9, 2048, 64), (300, 17, 2048, 16), (1100, 2, 4096, 64)]
+
+
+@pytest.mark.parametrize("tokens,topk,dim,tile_m", CASES)
+@pytest.mark.parametrize("out_dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("kept", [0, 11, 24])
+def test_one_call_equals_two_steps(gpu, tokens, topk, dim, tile_m, out_dtype, kept):
+    experts, inter = 24, 256
+    p, meta, blocks = _problem(tokens, topk, dim, inter, experts, tile_m, kept, gpu)
+    kw = dict(model_dim=dim, inter_dim=inter, experts=experts, topk=topk, tile_m=tile_m, tile_n=128, tile_k=128,
+              doweight_stage2=True, in_dtype="fp8", out_dtype=out_dtype)
+    args = _args(p, meta, tokens, dim, inter, blocks)
+    rows = torch.zeros(tokens * topk * dim, dtype=_DT[out_dtype], device=gpu)
+    want = torch.empty(tokens * dim, dtype=_DT[out_dtype], device=gpu)
+    stream = torch.cuda.current_stream()
+    compile_moe_gemm2(**kw, accumulate=False)(rows, *args, stream)
+    compile_moe_reduction(topk=topk, model_dim=dim, dtype_str=out_dtype)(rows, want, None, tokens, stream)
+    # memory that the allocator hands out next holds NaNs: rows that are neither written nor zeroed show
+    n = rows.numel()
+    del rows
+    junk = torch.full((2 * n + 65536,), float("nan"), dtype=_DT[out_dtype], device=gpu)
+    del junk
+    got = torch.empty_like(want)
+    compile_moe_gemm2_ex(**kw, mode=MoeGemm2Mode.REDUCE)(got, *args, stream=stream)
+    assert torch.equal(got, want)
+
+
+def test_other_stream(gpu):
+    """Called for another stream than the current one: everything runs there."""
+    tokens, topk, dim = 1025, 8, 1024
+    p, meta, blocks = _problem(tokens, topk, dim, 256, 24, 32, 11, gpu)
+    s2 = compile_moe_gemm2_ex(model_dim=dim, inter_dim=256, experts=24, topk=topk, tile_m=32, tile_n=128, tile_k=128,
+                              doweight_stage2=True, in_dtype="fp8", out_dtype="f16", mode=MoeGemm2Mode.REDUCE)
+    args = _args(p, meta, tokens, dim, 256, blocks)
+    want, got = (torch.empty(tokens * dim, dtype=torch.float16, device=gpu) for _ in range(2))
+    s2(want, *args)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    s2(got, *args, stream=side)
+    side.synchronize()
+    assert torch.equal(got, want)
+    got.zero_()
+    torch.cuda.synchronize()
+    s2(got, *args, stream=side.cuda_stream)
+    side.synchronize()
+    assert torch.equal(got, want)
