@@ -510,31 +510,45 @@ int launch(int kind, int epi, int out_dtype, int variant, const GemmArgs& args, 
 // ---- per-row quantization ------------------------------------------------------------
 typedef void (*QuantFn)(QuantArgs);
 
-// registers-resident variant for rows of up to 1, 2, 4 or 8 slices, streaming beyond
-template <int IN, int OUT, int MODE, int NT>
-QuantFn quant_fn(int nslices) {
-  if (nslices <= 1) return quant_rows_kernel<IN, OUT, MODE, 1, NT>;
-  if (nslices <= 2) return quant_rows_kernel<IN, OUT, MODE, 2, NT>;
-  if (nslices <= 4) return quant_rows_kernel<IN, OUT, MODE, 4, NT>;
-  if (nslices <= 8) return quant_rows_kernel<IN, OUT, MODE, 8, NT>;
-  return quant_rows_kernel<IN, OUT, MODE, 0, NT>;
+// A quant launch: kernel, rows per workgroup and threads
+struct QuantLaunch {
+  QuantFn fn;
+  int rows, threads;
+};
+
+// Short rows: the lanes of one wave per row.  Else one workgroup per row, in registers for rows of
+// up to 1, 2, 4 or 8 slices, streaming beyond (quant_rows.h has the rules' figures).
+template <int IN, int OUT, int MODE>
+QuantLaunch quant_fn(int M, int N) {
+#define SHORT(LPR, VPT) \
+  if (N <= LPR * 8 * VPT) return QuantLaunch{quant_short_rows_kernel<IN, OUT, MODE, LPR, VPT>, 256 / LPR, 256};
+  SHORT(8, 1) SHORT(16, 1) SHORT(32, 1) SHORT(64, 1)
+  if (M >= kQuantManyRows) {
+    SHORT(64, 2) SHORT(64, 4)
+  }
+#undef SHORT
+  auto pick = [&](auto nt) -> QuantLaunch {
+    constexpr int NT = decltype(nt)::value;
+    const int nslices = (N + NT * 8 - 1) / (NT * 8);
+    QuantFn fn = nslices <= 1   ? quant_rows_kernel<IN, OUT, MODE, 1, NT>
+                 : nslices <= 2 ? quant_rows_kernel<IN, OUT, MODE, 2, NT>
+                 : nslices <= 4 ? quant_rows_kernel<IN, OUT, MODE, 4, NT>
+                 : nslices <= 8 ? quant_rows_kernel<IN, OUT, MODE, 8, NT>
+                                : quant_rows_kernel<IN, OUT, MODE, 0, NT>;
+    return QuantLaunch{fn, 1, NT};
+  };
+  if (N >= kQuantWideN || M <= kQuantFewRows) return pick(std::integral_constant<int, 512>{});
+  return pick(std::integral_constant<int, 256>{});
 }
 
-template <int IN, int NT>
-QuantFn quant_fn_in(int out_dtype, int mode, int nslices) {
+template <int IN>
+QuantLaunch quant_fn_in(int out_dtype, int mode, int M, int N) {
   if (out_dtype == QOUT_FP8)
-    return mode == QMODE_DIV_NEAREST ? quant_fn<IN, QOUT_FP8, QMODE_DIV_NEAREST, NT>(nslices) : nullptr;
-  if (mode == QMODE_RECIP_TRUNC) return quant_fn<IN, QOUT_INT8, QMODE_RECIP_TRUNC, NT>(nslices);
-  if (mode == QMODE_DIV_TRUNC) return quant_fn<IN, QOUT_INT8, QMODE_DIV_TRUNC, NT>(nslices);
-  if (mode == QMODE_DIV_NEAREST) return quant_fn<IN, QOUT_INT8, QMODE_DIV_NEAREST, NT>(nslices);
-  return nullptr;
-}
-
-template <int NT>
-QuantFn quant_fn_nt(int in_dtype, int out_dtype, int mode, int nslices) {
-  return in_dtype == FLYGEMM_QIN_F16    ? quant_fn_in<QIN_F16, NT>(out_dtype, mode, nslices)
-         : in_dtype == FLYGEMM_QIN_BF16 ? quant_fn_in<QIN_BF16, NT>(out_dtype, mode, nslices)
-                                        : quant_fn_in<QIN_F32, NT>(out_dtype, mode, nslices);
+    return mode == QMODE_DIV_NEAREST ? quant_fn<IN, QOUT_FP8, QMODE_DIV_NEAREST>(M, N) : QuantLaunch{nullptr, 0, 0};
+  if (mode == QMODE_RECIP_TRUNC) return quant_fn<IN, QOUT_INT8, QMODE_RECIP_TRUNC>(M, N);
+  if (mode == QMODE_DIV_TRUNC) return quant_fn<IN, QOUT_INT8, QMODE_DIV_TRUNC>(M, N);
+  if (mode == QMODE_DIV_NEAREST) return quant_fn<IN, QOUT_INT8, QMODE_DIV_NEAREST>(M, N);
+  return QuantLaunch{nullptr, 0, 0};
 }
 
 // K in bytes for the kernels, which take K tiles of 128 bytes and a last tile of 64 bytes
@@ -623,13 +637,12 @@ int flygemm_quant_rows(void* out, float* scales, const void* in, int32_t M, int3
   if (!out || !scales || !in) return fail(hipErrorInvalidValue, "null pointer");
   if (((uintptr_t)in & 15) || ((uintptr_t)out & 7) || ((uintptr_t)scales & 3))
     return fail(hipErrorInvalidValue, "misaligned pointer (input needs 16-byte, output 8-byte alignment)");
-  const int nt = N >= kQuantWideN ? 2 * kQuantThreads : kQuantThreads;
-  const int nslices = (N + nt * 8 - 1) / (nt * 8);
-  QuantFn fn = nt == kQuantThreads ? quant_fn_nt<kQuantThreads>(in_dtype, out_dtype, mode, nslices)
-                                   : quant_fn_nt<2 * kQuantThreads>(in_dtype, out_dtype, mode, nslices);
-  if (!fn) return fail(hipErrorInvalidValue, "unsupported quant combination");
+  const QuantLaunch q = in_dtype == FLYGEMM_QIN_F16    ? quant_fn_in<QIN_F16>(out_dtype, mode, M, N)
+                        : in_dtype == FLYGEMM_QIN_BF16 ? quant_fn_in<QIN_BF16>(out_dtype, mode, M, N)
+                                                       : quant_fn_in<QIN_F32>(out_dtype, mode, M, N);
+  if (!q.fn) return fail(hipErrorInvalidValue, "unsupported quant combination");
   QuantArgs args{out, scales, in, M, N};
-  hipLaunchKernelGGL(fn, dim3(M), dim3(nt), 0, (hipStream_t)stream, args);
+  hipLaunchKernelGGL(q.fn, dim3((unsigned)(((long)M + q.rows - 1) / q.rows)), dim3(q.threads), 0, (hipStream_t)stream, args);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(e, "launch of quant_rows failed: %s", hipGetErrorString(e));
   return 0;

@@ -1,0 +1,72 @@
+"""Row quantization at the edges of their kernels: every lanes-per-row form and its first
+longer row, both workgroup sizes, row counts that fill no workgroup, and rows whose quotients take the
+reciprocal form, the division (scales outside 2^-90 .. 2^90) and the scrubbing of NaN and infinity.
+Codes and scales bit for bit against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from flydsl_amd.kernels.quant import build_quant_module, per_token_quant
+from flydsl_amd.quant import FP8
+from oracle import quant as oq
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(N, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(29, N, generator=g) * torch.exp(3 * torch.randn(29, 1, generator=g))
+    x[1] = 0.0
+    x[2] = -0.0
+    x[3, ::2] = -0.0
+    x[4] *= 1e-30          # bf16 / fp32: scales below 2^-90, or zero in fp16
+    x[5] *= 1e-38
+    x[6, N // 2] = float("inf")
+    x[7, N - 1] = float("nan")
+    x[8, 0], x[8, N // 3] = -float("inf"), float("nan")
+    if dtype != torch.float16:
+        x[9] *= 1e30
+    x[10] = torch.round(x[10])
+    return x.to(dtype)
+
+
+EDGES = [8, 64, 72, 128, 136, 256, 264, 512, 520, 1024, 1032, 2048, 2056, 4096, 8184, 8192]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("qd,rounding", [(torch.int8, "nearest"), (torch.int8, "trunc"), (FP8, "nearest")])
+def test_rows(gpu, dtype, qd, rounding):
+    for N in EDGES:
+        x = _rows(N, dtype, N)
+        q_ref, s_ref = oq.quant_rows(x.float().numpy(), "fp8" if qd == FP8 else "int8",
+                                     rounding="truncate" if rounding == "trunc" else "nearest")
+        q_ref, s_ref = q_ref.view(np.uint8), s_ref.view(np.uint32)
+        for copies, extra in ((1, 0), (36, 3), (142, 1)):   # 29, 1047 and 4119 rows
+            xb = torch.cat([x.repeat(copies, 1), x[:extra]]).to(gpu)
+            q, s = per_token_quant(xb, quant_dtype=qd, rounding=rounding)
+            rows = np.arange(xb.shape[0]) % 29
+            assert np.array_equal(s.cpu().view(-1).numpy().view(np.uint32), s_ref.reshape(-1)[rows]), (N, copies)
+            assert np.array_equal(q.cpu().view(torch.uint8).numpy(), q_ref[rows]), (N, copies)
+
+
+def test_reference_kernel_form(gpu):
+    for N in EDGES:
+        x = _rows(N, torch.float16, N)[:6]
+        q_ref, s_ref = oq.quant_rows_recip(x.numpy())
+        launch, _ = build_quant_module(N)
+        q = torch.empty(6, N, dtype=torch.int8, device=gpu)
+        s = torch.empty(6, dtype=torch.float32, device=gpu)
+        launch(x.to(gpu), q, s, 6)
+        assert np.array_equal(s.cpu().numpy().view(np.uint32), s_ref.reshape(-1).view(np.uint32))
+        assert np.array_equal(q.cpu().numpy(), q_ref)
+
+
+def test_quotients_are_the_divisions(gpu):
+    """fp32 rows of random significands: codes of x / scale with the division that torch makes."""
+    g = torch.Generator(device=gpu).manual_seed(0)
+    x = torch.randn(4096, 2048, generator=g, device=gpu) * torch.exp(8 * torch.randn(4096, 1, generator=g, device=gpu))
+    for qd in (FP8, torch.int8):
+        q, s = per_token_quant(x, quant_dtype=qd)
+        y = x / s
+        want = y.to(FP8) if qd == FP8 else torch.round(y).clamp_(-127, 127).to(torch.int8)
+        assert torch.equal(q.view(torch.uint8), want.view(torch.uint8))
