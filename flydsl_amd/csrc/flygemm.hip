@@ -648,6 +648,25 @@ int flygemm_quant_rows(void* out, float* scales, const void* in, int32_t M, int3
   return 0;
 }
 
+int flygemm_quant_blocks(void* out, float* scales, const void* in, int64_t blocks, int32_t in_dtype, float qmax,
+                         void* stream) {
+  if (blocks < 0 || blocks >= (1L << 35)) return fail(hipErrorInvalidValue, "invalid block count %ld", (long)blocks);
+  if (in_dtype < FLYGEMM_QIN_F16 || in_dtype > FLYGEMM_QIN_F32)
+    return fail(hipErrorInvalidValue, "quant in_dtype %d not supported", in_dtype);
+  if (blocks == 0) return 0;
+  if (!out || !scales || !in) return fail(hipErrorInvalidValue, "null pointer");
+  if (((uintptr_t)in & 15) || ((uintptr_t)out & 7) || ((uintptr_t)scales & 3))
+    return fail(hipErrorInvalidValue, "misaligned pointer (input needs 16-byte, output 8-byte alignment)");
+  BlockQuantArgs args{out, scales, in, blocks, 1.f / qmax};
+  auto fn = in_dtype == FLYGEMM_QIN_F16    ? quant_blocks_kernel<QIN_F16>
+            : in_dtype == FLYGEMM_QIN_BF16 ? quant_blocks_kernel<QIN_BF16>
+                                           : quant_blocks_kernel<QIN_F32>;
+  hipLaunchKernelGGL(fn, dim3((unsigned)((blocks + 15) / 16)), dim3(256), 0, (hipStream_t)stream, args);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(e, "launch of quant_blocks failed: %s", hipGetErrorString(e));
+  return 0;
+}
+
 int flygemm_preshuffle_quant_a(void* c, void* a_q, float* scale_a, const void* x, const void* b, const float* scale_b,
                                int32_t M, int32_t N, int32_t K, int32_t x_dtype, int32_t in_dtype, int32_t mode,
                                int32_t out_dtype, int32_t variant, void* stream) {

@@ -358,4 +358,65 @@ __global__ void __launch_bounds__(NT) quant_rows_kernel(QuantArgs p) {
   }
 }
 
+// One scale per 128 consecutive elements of a row (blockscale activations), fp8 codes:
+//   scale = amax * inv_qmax (1 where that is 0), code = e4m3fn(x / scale),
+// the arithmetic of torch's operators on the GPU, where a division by a constant is a product
+// with its reciprocal, amax passes NaN on, and the cast keeps NaN's sign.
+// 16 lanes per block of 128, each with 8 elements; bound by HBM for many blocks and by its launch
+// for few (torch.float16, back-to-back calls from Python: 1024 x 7168 14.9 us against 58.5
+// for the operators, 65536 x 256 14.1 against 104).
+struct BlockQuantArgs {
+  void* out;        // [blocks][128] fp8 codes
+  float* scales;    // [blocks]
+  const void* in;   // [blocks][128]
+  long blocks;
+  float inv_qmax;
+};
+
+template <int IN>
+__global__ void __launch_bounds__(256) quant_blocks_kernel(BlockQuantArgs p) {
+  constexpr int ESZ = (IN == QIN_F32) ? 4 : 2;
+  const int lane = threadIdx.x % 16;
+  const long blk = (long)blockIdx.x * 16 + threadIdx.x / 16;
+  if (blk >= p.blocks) return;   // whole groups of 16 lanes
+  Raw8<IN> raw;
+  raw.load((const uint8_t*)p.in + (size_t)blk * 128 * ESZ, lane * 8);
+  uint32_t mb = Raw8<IN>::fold(raw.max_bits(0));
+#pragma unroll
+  for (int off = 8; off >= 1; off >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, off, 64));
+  const bool finite = mb < Raw8<IN>::kInf;
+  float scale = Raw8<IN>::abs_value(mb) * p.inv_qmax;
+  if (scale == 0.f) scale = 1.f;
+  const f32x8 v = raw.value();
+  if (mb > Raw8<IN>::kInf) {   // NaN: the block's first one
+    uint32_t first = 0;
+    bool nan = false;
+#pragma unroll
+    for (int i = 7; i >= 0; --i) {
+      const float x = v[i];
+      if (x != x) {
+        nan = true;
+        first = __builtin_bit_cast(uint32_t, x);
+      }
+    }
+    const uint64_t m = (__builtin_amdgcn_ballot_w64(nan) >> (threadIdx.x & 48)) & 0xFFFFu;
+    first = (uint32_t)__shfl((int)first, (threadIdx.x & 48) + __builtin_ctzll(m), 64);
+    scale = __builtin_bit_cast(float, first | 0x00400000u);   // quiet, its payload kept
+  }
+  if (lane == 0) p.scales[blk] = scale;
+  uint2 c = quant8<QOUT_FP8, QMODE_DIV_NEAREST>(v, scale, 1.f / scale, div_by_ok(scale));
+  if (!finite) {
+    uint32_t w[2] = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float y = v[i] / scale;
+      const uint32_t b = __builtin_bit_cast(uint32_t, y);
+      const uint32_t code = (b >> 24 & 0x80u) | (y != y ? 0x7Fu : 0u);   // finite / infinite = 0
+      w[i / 4] |= code << (8 * (i % 4));
+    }
+    c = make_uint2(w[0], w[1]);
+  }
+  store8((uint8_t*)p.out + (size_t)blk * 128 + lane * 8, c);
+}
+
 }  // namespace flygemm

@@ -21,20 +21,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-
-
-def _plain_cuda(*ts) -> bool:
-    """Tensors whose values a kernel may read and write by pointer in place of torch's own
-    operators: ordinary tensors of one GPU, outside autograd, functorch, tracing and dispatch modes."""
-    dev = ts[0].device
-    if dev.type != "cuda" or any(type(t) is not torch.Tensor or t.device != dev for t in ts):
-        return False
-    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
-        return False
-    C = torch._C
-    return not (C._len_torch_dispatch_stack() or C._len_torch_function_stack() or torch.compiler.is_compiling()
-                or C._get_tracing_state() is not None or C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0)
+from ._tensors import on_device, plain_cuda
 
 
 def _sort_kernel(topk_ids, topk_weights, E, bs, expert_mask):
@@ -78,10 +65,8 @@ def moe_sorting(topk_ids: torch.Tensor, topk_weights: torch.Tensor, num_experts:
     # the buffers), empty routings and masks shorter than the experts take the operators below.
     if (0 < topk <= E <= _lib.MOE_SORT_MAX_EXPERTS and M > 0 and max_pad < 2**31 - 2**16
             and (expert_mask is None or expert_mask.numel() >= E)
-            and _plain_cuda(*(t for t in (topk_ids, topk_weights, expert_mask) if t is not None))):
-        if dev.index == torch.cuda.current_device():
-            return _sort_kernel(topk_ids, topk_weights, E, bs, expert_mask)
-        with torch.cuda.device(dev):
+            and plain_cuda(*(t for t in (topk_ids, topk_weights, expert_mask) if t is not None))):
+        with on_device(dev):
             return _sort_kernel(topk_ids, topk_weights, E, bs, expert_mask)
     max_blocks = (max_pad + bs - 1) // bs
 

@@ -107,6 +107,13 @@ enum { FLYGEMM_QMODE_RECIP_TRUNC = 0, FLYGEMM_QMODE_DIV_TRUNC = 1, FLYGEMM_QMODE
 int flygemm_quant_rows(void* out, float* scales, const void* in, int32_t M, int32_t N, int32_t in_dtype,
                        int32_t out_dtype, int32_t mode, void* stream);
 
+/* fp8 codes and scales of blocks of 128 consecutive elements (the activations of the blockscale
+ * GEMMs, flydsl_amd.quant.blockscale_quant with 1 x 128 blocks): scales[b] = amax * (1 / qmax), 1
+ * where that is 0, out = e4m3fn(in / scale), in fp32; NaN and infinity propagate.  qmax at most 448;
+ * in_dtype as for flygemm_quant_rows; in 16-byte, out 8-byte aligned. */
+int flygemm_quant_blocks(void* out, float* scales, const void* in, int64_t blocks, int32_t in_dtype, float qmax,
+                         void* stream);
+
 /* The GEMM of activations quantized per row on the way in, in one call:
  *   flygemm_quant_rows(a_q, scale_a, x, M, K, x_dtype, fp8 or int8 codes, mode), then
  *   flygemm_preshuffle(c, a_q, b, scale_a, scale_b, M, N, K, in_dtype, out_dtype, variant)

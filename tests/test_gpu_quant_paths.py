@@ -1,13 +1,13 @@
-"""Row quantization at the edges of their kernels: every lanes-per-row form and its first
+"""Row and block quantization at the edges of their kernels: every lanes-per-row form and its first
 longer row, both workgroup sizes, row counts that fill no workgroup, and rows whose quotients take the
 reciprocal form, the division (scales outside 2^-90 .. 2^90) and the scrubbing of NaN and infinity.
-Codes and scales bit for bit against the oracle."""
+Codes and scales bit for bit against the oracle (rows) and torch's operators on the GPU (blocks)."""
 import numpy as np
 import pytest
 import torch
 
 from flydsl_amd.kernels.quant import build_quant_module, per_token_quant
-from flydsl_amd.quant import FP8
+from flydsl_amd.quant import FP8, blockscale_quant
 from oracle import quant as oq
 
 pytestmark = pytest.mark.gpu
@@ -70,3 +70,35 @@ def test_quotients_are_the_divisions(gpu):
         y = x / s
         want = y.to(FP8) if qd == FP8 else torch.round(y).clamp_(-127, 127).to(torch.int8)
         assert torch.equal(q.view(torch.uint8), want.view(torch.uint8))
+
+
+def _block_ops(x, qmax):
+    R, C = x.shape
+    t = x.to(torch.float32).view(R, C // 128, 128)
+    amax = torch.maximum(t.amax(dim=-1, keepdim=True), -t.amin(dim=-1, keepdim=True))
+    scale = amax / qmax
+    scale[scale == 0] = 1
+    return (t / scale).reshape(R, C).to(FP8), scale.reshape(R, C // 128)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("R,C", [(1, 128), (3, 384), (29, 1024), (515, 7168)])
+@pytest.mark.parametrize("qmax", [448.0, 240])
+def test_blocks(gpu, dtype, R, C, qmax):
+    x = _rows(C, dtype, R)[:R].repeat((R + 28) // 29, 1)[:R].to(gpu)
+    for y in (x, x.t().contiguous().t(), torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(R, C)):   # strided, unaligned
+        q, s = blockscale_quant(y, 1, 128, qmax)
+        q_ref, s_ref = _block_ops(x, qmax)
+        assert q.shape == (R, C) and s.shape == (R, C // 128) and s.is_contiguous()
+        assert torch.equal(s.view(torch.int32), s_ref.view(torch.int32))
+        assert torch.equal(q.view(torch.uint8), q_ref.view(torch.uint8))
+
+
+def test_blocks_keep_the_operators(gpu):
+    """Under autograd, and for a code range past the type's, the operators run as before."""
+    x = torch.randn(4, 256, device=gpu, requires_grad=True)
+    _, s = blockscale_quant(x, 1, 128)
+    s.sum().backward()
+    assert x.grad is not None and int((x.grad != 0).sum()) == 8
+    q, _ = blockscale_quant(x.detach(), 1, 128, 1000.0)
+    assert torch.equal(q.view(torch.uint8), _block_ops(x.detach(), 1000.0)[0].view(torch.uint8))
