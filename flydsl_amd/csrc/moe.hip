@@ -17,7 +17,7 @@ using namespace flygemm;
 // of blockscale fp8 -- runs of one routing block (R = 1, 4 waves) for every (tile_m, tile_n).
 namespace flygemm {
 MoeKernel moe_stage2_kernel(int kind, int tm, int r, int tn, bool f32, bool bs);
-MoeKernel moe_stage1_stream_kernel(int kind, int tm);
+MoeKernel moe_stage1_stream_kernel(int kind, int tm, bool bs, bool gs);
 MoeKernel moe_stage2_stream_kernel(int kind, int tm, int nk, bool single);
 }
 
@@ -37,10 +37,6 @@ MoeKernel moe_stage1_tile(int tm, int r, int tn) {
   }
   if constexpr (KIND == KIND_W4A16) {
     T(64, 4, 128, 2, 4) T(32, 8, 128, 2, 4)
-  }
-  // blockscale with 16-row blocks: runs of 256 rows, 64 columns (see moe_tiles)
-  if constexpr (BS) {
-    T(16, 16, 64, 2, 4)
   }
 #undef T
   return MoeKernel{nullptr, 0};
@@ -73,7 +69,7 @@ MoeKernel moe_stage1_kernel(int kind, int tm, int r, int tn, bool bs) {
     }
   }
   if (moe_stream_stage1(1, kind, bs))
-    return r * tm == 128 && tn == 64 ? moe_stage1_stream_kernel(kind, tm) : MoeKernel{nullptr, 0};
+    return r * tm == 128 && tn == 64 ? moe_stage1_stream_kernel(kind, tm, false, false) : MoeKernel{nullptr, 0};
   return kind == KIND_W4A16 ? moe_stage1_tile<KIND_W4A16, false>(tm, r, tn) : MoeKernel{nullptr, 0};
 }
 
@@ -233,6 +229,26 @@ int moe_tiles(int stage, int tokens, int N, int K, int experts, int topk, int ti
   return 0;
 }
 
+// Stage 1 of W4A16 and of blockscale on the stream kernel (runs of 64 and 128 rows, 64 columns), in
+// place of moe_tiles' LDS-staged tiles.  Those re-read the weights for every 16 to 64 rows and have
+// one 128-byte K tile in flight, of which W4A16's share of the weights is 1 KB per 16 columns.
+// Graph-timed on MI355X (us, the LDS-staged choice against this kernel; blockscale bit-equal):
+//   W4A16, per-row scales: 7168 x 256, 128 experts, top-8: 4 / 256 / 2048 / 8192 tokens, 16-row
+//   blocks 53.3 / 108.5 / 530 / 1583 against 42.4 / 92.1 / 176 / 540, 64-row blocks 63.9 / 72.6 / 240 /
+//   711 against 41.6 / 60.9 / 172 / 521; 4096 x 14336, 8 experts, top-2: 1 / 32 / 600 / 3000 tokens,
+//   64-row blocks 43.3 / 161 / 474 / 1902 (runs of 256 rows) against 37.0 / 128 / 408 / 1669.  Its steps
+//   are four K tiles of A, so K must be a multiple of 256 elements.
+//   Group scales gain alike (6144 x 1024, 128 experts, 1000 tokens, 32-row blocks 760 against 454) but
+//   with fewer than 4 routes per expert (4096 x 2048, 17 experts, 4 tokens 66.5 against 70.2).
+//   Blockscale, 64-row blocks: 7168 x 256, 256 experts, 2 / 4 / 31 / 125 routes per expert 106 / 166 / 243
+//   / 368 against 128 / 145 / 194 / 283; 32-row: 4 / 8 / 31 / 125 routes 147 / 150 / 238 / 538 against 146 /
+//   150 / 198 / 296; 4096 x 1536, 64 experts, 16-row blocks, 8 / 16 / 31 / 62 / 250 / 750 routes 141 / 146 /
+//   217 / 361 / 766 / 1767 against 151 / 168 / 167 / 192 / 402 / 915.
+bool moe_stage1_streams(int kind, bool bs, bool gs, int tile_m, int kb, long routes, long experts) {
+  if (bs) return routes >= (tile_m == 64 ? 4 : 24) * experts;
+  return kind == KIND_W4A16 && kb % 512 == 0 && (!gs || routes >= 4 * experts);
+}
+
 // in_dtype -> kernel kind (and whether stage-1 activations come per route); -1 if unknown
 int moe_kind(int in_dtype, int stage, bool* token_slot) {
   *token_slot = false;
@@ -356,6 +372,12 @@ int moe_plan(int stage, void* out, const void* a, const void* w, const float* sa
       }
     }
   }
+  const bool stream1 = stage == 1 && moe_stage1_streams(kind, bs, group_size > 0, tile_m, (int)kb, routes_all, experts);
+  if (stream1) {
+    k = moe_stage1_stream_kernel(kind, tile_m, bs, group_size > 0);
+    R = (kind == KIND_W4A16 ? 64 : 128) / tile_m;
+    tile_n = 64;
+  }
   if (!k.fn) return fail(hipErrorInvalidValue, "%s: no kernel for tile %dx%d (runs of %d)", what, tile_m, tile_n, R);
 
   // column ranges per run: about 1024 workgroups in all (the stream kernel: one column tile each)
@@ -363,7 +385,7 @@ int moe_plan(int stage, void* out, const void* a, const void* w, const float* sa
   const long runs = est_runs(tokens, topk, experts, tile_m, R);
   long nsplit = (1024 + runs - 1) / runs;
   nsplit = nsplit < 1 ? 1 : (nsplit > ntn ? ntn : nsplit);
-  if (moe_stream_stage1(stage, kind, bs)) nsplit = ntn;
+  if (moe_stream_stage1(stage, kind, bs) || stream1) nsplit = ntn;
   // stage 2 with atomics: at least half as many column ranges as tiles (two tiles of 128 columns
   // or 256 per workgroup, at most; about 1024 workgroups leave few runs long walks whose atomic
   // epilogues queue behind each other).  Graph-timed, fp8 (blockscale for DS-V3-M128), the
