@@ -88,6 +88,12 @@ int pick_tile_n(int N, long runs) {
   return 64;
 }
 
+// Routings with large experts (moe_tiles has the figures)
+bool moe_large_experts(int kind, int inter, long routes, long experts) {
+  return kind == KIND_INT4 ? inter >= 4096 && routes >= 512L * experts
+                           : (inter >= 1024 && routes >= 512L * experts) || (inter >= 4096 && routes >= 256L * experts);
+}
+
 // Tile of a call: runs of R routing blocks per workgroup and tile_n output columns (the
 // caller's tile_n, already validated, is a hint).  atomics: a stage-2 call that accumulates
 // (per-route-row calls take the stream kernel's tiles where it applies).
@@ -144,9 +150,7 @@ int moe_tiles(int stage, int tokens, int N, int K, int experts, int topk, int ti
   // 4096 x 14336, 8 experts, top-2: 485 -> 361 / 358 -> 199; 1024 tokens, 8192 x 8192, 16
   // experts, top-4: 1148 -> 906 / 816 -> 478), not at 1536 (2048 tokens, 64 experts, top-8, stage
   // 2 256 -> 265) nor with fewer routes (128 per expert, 4096 x 1536: 198 -> 216 / 155 -> 210).
-  const bool big = kind == KIND_INT4 ? inter >= 4096 && routes >= 512L * experts
-                                     : (inter >= 1024 && routes >= 512L * experts) ||
-                                           (inter >= 4096 && routes >= 256L * experts);
+  const bool big = moe_large_experts(kind, inter, routes, experts);
   // W4A16 with per-row weight scales (no group scales, which ride the two-slot pipeline) takes
   // them as bf16 does, for 32- and 64-row blocks (4096 tokens, 8192 x 8192, 16 experts, top-4:
   // 6994 -> 5431 / 3271 -> 2392; 8192 tokens, 4096 x 14336, 8 experts, top-2: 6213 -> 4603 / 2780
@@ -247,6 +251,47 @@ int moe_tiles(int stage, int tokens, int N, int K, int experts, int topk, int ti
 bool moe_stage1_streams(int kind, bool bs, bool gs, int tile_m, int kb, long routes, long experts) {
   if (bs) return routes >= (tile_m == 64 ? 4 : 24) * experts;
   return kind == KIND_W4A16 && kb % 512 == 0 && (!gs || routes >= 4 * experts);
+}
+
+// Stage 2 of routings between decode and the 256-row runs of large experts: runs of 64 rows (32) on
+// the 4-wave tiles, where moe_tiles takes 256-row runs of 16-row blocks from 32 routes per expert,
+// most of them empty, or single blocks that each re-read their expert's weights.  r: moe_tiles' run.
+// Graph-timed on MI355X (us; moe_tiles' choice against 64 rows x 128 columns unless said):
+//   * 16-row blocks, inter_dim of less than 1024 bytes, atomics: from 64 routes per expert (7168 x 256:
+//     94 routes 577 against 326, 250: 500 against 389, 512: 880 against 760; bf16 250: 576 against 438);
+//     from 32, 32 rows x 64 columns (40 routes 478 against about 155; 188 with 64 rows).
+//   * deeper inter_dims (at least 1024 bytes).  16-row blocks from 32 routes per expert (4096 x 1536
+//     int8, 37 / 75 / 187 routes: atomics 173 / 236 / 255 against 90 / 114 / 198, rows 150 / 192 / 210
+//     against 108 / 132 / 221; 4096 x 14336 fp8, 37 / 75 / 175: 168 / 329 / 342 against 110 / 142 / 268).
+//     32-row blocks, atomics, the same (95 / 129 / 277 against 90 / 112 / 190; 167 / 170 / 297 against 110 /
+//     142 / 246; int4 6144 x 1024 at 62 routes 173 against 141); rows: single blocks of 128 columns
+//     (never 64: 4096 x 14336 at 37 routes 166 against 108) and 64-row runs from 128 routes (187 routes
+//     247 against 196, 175: 320 against 245; below that level or slower, as for int4: 135 against 161).
+//     64-row blocks, atomics: 128 columns in place of 64 from 48 routes (75 routes 118 against 113
+//     and 183 against 110, 187: 206 against 179; at 19 routes 78 against 90).
+//   * W4A16 and blockscale (single blocks in moe_tiles) from 48 routes: blockscale 4096 x 1536 at 125
+//     routes, 16- / 32-row blocks 288 / 250 against 183 / 181, W4A16 4096 x 14336 at 75 routes, 16-row
+//     blocks 351 against 210; at 31 routes and fewer slower.
+bool moe_stage2_mid(int kind, bool bs, bool rows, int tile_m, int r, int kb, int n, long routes, long experts,
+                    int* r_out, int* tn_out) {
+  if (n % 128 != 0) return false;
+  // moe_tiles' 256-row runs of large experts stay; 16-row blocks have runs from 32 routes per expert
+  const bool runs16 = !bs && kind != KIND_W4A16 && tile_m == 16;
+  const int inter = moe_a_16bit(kind) ? kb / 2 : kb;
+  if (r > 1 && !(runs16 && !moe_large_experts(kind, inter, routes, experts))) return false;
+  const bool deep = kb >= 1024;
+  const long from = bs || kind == KIND_W4A16 ? 48 : 32;
+  if (routes < from * experts || (!deep && !(runs16 && !rows))) return false;
+  if (tile_m == 64 && (rows || routes < 48 * experts)) return false;
+  const bool narrow = !deep && routes < 64 * experts;
+  *tn_out = narrow ? 64 : 128;
+  if (tile_m == 16)
+    *r_out = narrow ? 2 : 4;
+  else if (tile_m == 32)
+    *r_out = !rows || (routes >= 128 * experts && kind != KIND_INT4) ? 2 : 1;
+  else
+    *r_out = 1;
+  return true;
 }
 
 // in_dtype -> kernel kind (and whether stage-1 activations come per route); -1 if unknown
@@ -378,6 +423,9 @@ int moe_plan(int stage, void* out, const void* a, const void* w, const float* sa
     R = (kind == KIND_W4A16 ? 64 : 128) / tile_m;
     tile_n = 64;
   }
+  if (stage == 2 && !stream2 &&
+      moe_stage2_mid(kind, bs, rows, tile_m, R, (int)kb, N, routes_all, experts, &R, &tile_n))
+    k = moe_stage2_kernel(kind, tile_m, R, tile_n, mout == MOE_OUT_F32, bs);
   if (!k.fn) return fail(hipErrorInvalidValue, "%s: no kernel for tile %dx%d (runs of %d)", what, tile_m, tile_n, R);
 
   // column ranges per run: about 1024 workgroups in all (the stream kernel: one column tile each)

@@ -16,6 +16,11 @@ MoeKernel stage2_tile(int tm, int r, int tn) {
   // tiles of 256 columns (it narrows them to 128 or 64)
   T(16, 1, 64, 1, 4) T(16, 1, 128, 1, 4) T(32, 1, 64, 1, 4) T(32, 1, 128, 1, 4) T(64, 1, 64, 1, 4)
   T(64, 1, 128, 1, 4)
+  // runs of 64 rows, 128 columns, and of 32 rows, 64 columns (moe_stage2_mid)
+  T(16, 4, 128, 1, 4) T(32, 2, 128, 1, 4)
+  if constexpr (!BS && KIND != KIND_W4A16) {
+    T(16, 2, 64, 1, 4)
+  }
   // run tiles of 256 rows: for 16-row blocks only (32- and 64-row blocks keep single-block
   // tiles in stage 2); not for blockscale (its partials and factors do not fit next to them)
   // nor W4A16 (its group scales ride the two-slot pipeline)

@@ -216,7 +216,8 @@ int flygemm_moe_blockscale_gemm2(void* out, const void* a2, const void* w, const
  * with 1 to 32 routes per expert on average, 128-row runs from 128 routes per expert (int4: 256;
  * from 32 for tile_m 16).  Stage 1 of W4A16 with a model_dim of whole 256-element steps and of
  * blockscale leaves this choice for the stream kernel's runs (64 and 128 rows, 64 columns) at the
- * routes per expert that csrc/moe.hip names.  n is the GEMM's output width and k its depth (stage 1: inter_dim and
+ * routes per expert that csrc/moe.hip names, and stage 2 of routings between decode and large
+ * experts for runs of 32 and 64 rows.  n is the GEMM's output width and k its depth (stage 1: inter_dim and
  * model_dim; stage 2: model_dim and inter_dim); in_dtype as for flygemm_moe_gemm1/2; blockscale
  * != 0 for the blockscale MoE.  Validates like the launchers; touches no device.  Counterpart of
  * the reference's compile-time tile arguments (kernels/moe_gemm_2stage.py:93-121), for tests and

@@ -1,9 +1,12 @@
-"""MoE stage 1 of W4A16 and blockscale on the stream kernel, against the oracle at the bar of
-tests/test_gpu_moe.py: every number of K steps around its register sets, partly filled runs."""
+"""MoE stages on the tiles between decode and large experts, against the oracle at the bar of
+tests/test_gpu_moe.py: stage 1 of W4A16 and blockscale on the stream kernel (every number of K steps
+around its register sets, partly filled runs), and stage 2 on runs of 32 and 64 rows."""
 import pytest
 import torch
 
 from flydsl_amd import workloads as W
+from flydsl_amd.kernels.moe_gemm_2stage import MoeGemm2Mode, compile_moe_gemm2_ex
+from tests import helpers as H
 from tests import test_gpu_moe as M
 
 pytestmark = pytest.mark.gpu
@@ -31,12 +34,57 @@ def test_blockscale_stage1_stream(gpu, tile_m, tokens):
         M._check(out, M.ref_bs1(p, K % 256 == 0), what=f"blockscale tm{tile_m} t{tokens} K{K}")
 
 
+def _reduce(p, gpu, kind, out_dtype):
+    w = p["workload"]
+    fn = compile_moe_gemm2_ex(model_dim=w.model_dim, inter_dim=w.inter_dim, experts=w.experts, topk=w.topk,
+                              tile_m=w.tile_m, tile_n=w.tile_n2, tile_k=M._tile_k(kind), doweight_stage2=True, in_dtype=kind,
+                              out_dtype=out_dtype, mode=MoeGemm2Mode.REDUCE)
+    out = torch.full((w.tokens, w.model_dim), float("nan"), dtype=M.OUT_T[out_dtype], device=gpu)
+    empty = torch.empty(0, dtype=torch.float32, device=gpu)
+    fn(out, H.dev_flat(p["a2"], gpu), H.dev_flat(p["w2_shuf"], gpu), empty if p["sa2"] is None else p["sa2"],
+       empty if p["sw2"] is None else p["sw2"], p["sorted_ids"], p["sorted_expert_ids"], p["sorted_weights"],
+       p["num_valid_ids"], w.tokens, w.model_dim, w.inter_dim, p["blocks"])
+    return out
+
+
+# kind, inter_dim, tokens (top-2 of 5 experts: 40, 60 and 160 routes per expert)
+STAGE2 = [("fp8", 256, 100), ("fp8", 256, 400), ("bf16", 128, 100), ("bf16", 256, 400), ("int4", 256, 100), ("fp8", 1024, 100),
+          ("fp8", 1152, 400), ("int8", 1024, 150), ("int4", 1024, 400), ("fp16", 512, 150), ("bf16", 576, 400),
+          ("int4_bf16", 512, 150), ("int4_bf16", 1024, 400)]
+
+
+@pytest.mark.parametrize("kind,inter,tokens", STAGE2)
+@pytest.mark.parametrize("tile_m", [16, 32, 64])
+@pytest.mark.parametrize("model_dim", [256, 384])
+def test_stage2_mid(gpu, kind, inter, tokens, tile_m, model_dim):
+    w = W.moe_custom(tokens, model_dim, inter, 5, 2, tile_m, 64, 128, kind, seed=inter + tokens + tile_m)
+    p = W.moe_problem(w, gpu)
+    what = f"stage2 {kind} tm{tile_m} t{tokens} {model_dim}x{inter}"
+    for out_dtype in ("f16", "f32", "bf16"):
+        out = M.run_stage2(p, gpu, out_dtype, doweight=True)
+        M.check_stage2(p, out, True, what=f"{what} atomics {out_dtype}",
+                       atol_rms=M.BF16_ATOMIC_ATOL if out_dtype == "bf16" else 1e-2)
+    M.check_stage2(p, _reduce(p, gpu, kind, "bf16"), True, what=f"{what} rows", route_round="bf16")
+
+
+@pytest.mark.parametrize("tile_m", [16, 32, 64])
+@pytest.mark.parametrize("tokens", [150, 240])
+def test_blockscale_stage2_mid(gpu, tile_m, tokens):
+    w = W.moe_custom(tokens, 384, 1024, 5, 2, tile_m, 128, 128, "fp8_block", seed=tokens + tile_m)
+    p = W.moe_problem(w, gpu)
+    for out_dtype, mode in (("f16", "atomic"), ("f32", "atomic"), ("f16", "reduce")):
+        out = M.run_bs_stage2(p, gpu, out_dtype, doweight=True, mode=mode)
+        M._check(out, M.ref_bs2(p, True), what=f"blockscale stage2 tm{tile_m} t{tokens} {mode} {out_dtype}")
+
+
 def test_under_graph_capture(gpu):
-    """Captured once and replayed, each replay equal to the eager run."""
+    """Both stages of W4A16 and blockscale captured once and replayed, each replay equal to the eager
+    run (stage 1 and the fp32 rows have one order; stage 2 through the reduce mode)."""
     for kind in ("int4_bf16", "fp8_block"):
         w = W.moe_custom(200, 512, 1024, 5, 2, 16, 64, 128, kind, seed=3)
         p = W.moe_problem(w, gpu)
-        run = (lambda: (M.run_bs_stage1(p, gpu),)) if kind == "fp8_block" else (lambda: (M.run_stage1(p, gpu, "bf16"),))
+        run = (lambda: (M.run_bs_stage1(p, gpu), M.run_bs_stage2(p, gpu, mode="reduce"))) if kind == "fp8_block" else \
+            (lambda: (M.run_stage1(p, gpu, "bf16"), _reduce(p, gpu, kind, "bf16")))
         eager = [t.clone() for t in run()]
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
