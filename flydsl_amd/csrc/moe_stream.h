@@ -88,6 +88,7 @@ __global__ void __launch_bounds__(256, 2) moe_stream_kernel(MoeArgs p) {
   constexpr int SLOT = A_BYTES + (BS ? TME * 4 : 0);   // blockscale: the rows' scales of the step after A
   constexpr int LPS = NB * (W4 ? KS : 2) + (BS ? NB : 0) + (GS ? NB * KS : 0);   // weight (and weight scale) loads per wave per step
   constexpr int Lb = D - 1;
+  constexpr int PD = W4 ? 1 : 2;                       // row blocks that A fragments are read ahead of their MFMAs
   static_assert(TME % 64 == 0 && A_TILE % (1024 * NW) == 0 && D >= 3, "tile shape");
   __shared__ __attribute__((aligned(1024))) uint8_t ring[2 * SLOT];
 
@@ -252,9 +253,13 @@ __global__ void __launch_bounds__(256, 2) moe_stream_kernel(MoeArgs p) {
     if constexpr (BS)
       if (wave < TME / 64) dma4(rsrc_sa, st + A_BYTES + wave * 256, vsa, (uint32_t)s * (uint32_t)a_rows * 4u);
   };
-  // One K step from register set U and the A slot sA: row block by row block, the next row's A
-  // fragment read ahead of this row's MFMAs.  B is the MFMA's first operand, so each accumulator
-  // tile holds its 16x16 output block transposed.
+  // One K step from register set U and the A slot sA: row block by row block, A fragments read PD row
+  // blocks ahead of their MFMAs.  The MFMAs of one row block cover less than the latency of an LDS read
+  // that eight waves contend for; graph-timed, one block ahead against two (us; DS-TP8 dims, 128
+  // experts): int4 64 / 2048 / 8192 tokens 47.5 / 95.8 / 244 against 38.4 / 87.5 / 238, fp8 8 / 8192
+  // tokens 33.9 / 291 against 31.8 / 289, bf16 8192 tokens 605 against 593; three ahead level with two.
+  // W4A16, whose conversions stand between the reads, 60 against 62 (64 tokens).  B is the MFMA's first
+  // operand, so each accumulator tile holds its 16x16 output block transposed.
   auto compute = [&](auto u_tag, const uint8_t* slot) __attribute__((always_inline)) {
     constexpr int U = decltype(u_tag)::value;
 #pragma unroll
@@ -282,8 +287,9 @@ __global__ void __launch_bounds__(256, 2) moe_stream_kernel(MoeArgs p) {
           bh[h] = bw[U][h][1];
         }
       }
-      i32x4 alo, ahi;
-      load_a(0, alo, ahi);
+      i32x4 alo[PD + 1], ahi[PD + 1];
+#pragma unroll
+      for (int mi = 0; mi < PD; ++mi) load_a(mi, alo[mi], ahi[mi]);
       f32x4 part[2][NB];
       float sa_t[2];
       // blockscale: row mi's partials into the accumulators, scaled, once the next row's MFMAs are out
@@ -297,8 +303,9 @@ __global__ void __launch_bounds__(256, 2) moe_stream_kernel(MoeArgs p) {
       };
 #pragma unroll
       for (int mi = 0; mi < MR; ++mi) {
-        const i32x4 lo = alo, hi = ahi;
-        if (mi + 1 < MR) load_a(mi + 1, alo, ahi);
+        const i32x4 lo = alo[mi % (PD + 1)], hi = ahi[mi % (PD + 1)];
+        if (mi + PD < MR) load_a(mi + PD, alo[(mi + PD) % (PD + 1)], ahi[(mi + PD) % (PD + 1)]);
+        if constexpr (PD > 1) __builtin_amdgcn_sched_barrier(0);   // the read stays here
         if constexpr (BS) sa_t[mi & 1] = *(const float*)(slot + A_BYTES + (mi * 16 + l16) * 4);
 #pragma unroll
         for (int h = 0; h < NB; ++h) {
