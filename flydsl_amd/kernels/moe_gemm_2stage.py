@@ -37,6 +37,8 @@ reference validates it and otherwise a hint (the kernels' K tile is 128 bytes).
 """
 from __future__ import annotations
 
+import contextlib
+
 import torch
 
 from .. import _lib
@@ -216,17 +218,28 @@ class MoeGemm2Mode:
     REDUCE = "reduce"       # per-route rows [tokens*topk, model_dim], then a reduction over topk
 
 
+def _on_stream(stream, handle, device):
+    """A context in which torch allocates and copies on the stream of a launcher's call."""
+    if handle == torch.cuda.current_stream(device).cuda_stream:
+        return contextlib.nullcontext()
+    if isinstance(stream, torch.cuda.Stream):
+        return torch.cuda.stream(stream)
+    return torch.cuda.stream(torch.cuda.ExternalStream(handle, device) if handle else torch.cuda.default_stream(device))
+
+
 class _MoeGemm2ReduceWrapper:
     """Stage 2 in reduce mode (reference ``moe_gemm_2stage.py:2689-2774``): the GEMM writes
     every route's row of an intermediate with plain stores, then the reduction sums the top-k rows
     of each token into ``arg_out``; one call to the library (``flygemm_moe_gemm2_reduce``).  The
-    intermediate comes from torch's caching allocator.  A route without a row adds nothing: a valid
-    mask says which rows to read, or ``zero_intermediate=False`` promises that every route is
-    written, or else the library finds them itself."""
+    intermediate comes from torch's caching allocator, from the pool of the stream that the call
+    runs on.  A route without a row adds nothing: a valid mask says which rows to read, or
+    ``zero_intermediate=False`` promises that every route is written, or else the library finds
+    them itself.  ``reduce_exe`` is the reference's argument; the library call holds its own
+    reduction, so compiling one only checks the reduction's sizes and type."""
 
     def __init__(self, gemm2_exe, reduce_exe, topk, model_dim, out_dtype_str="f16", use_mask=False,
                  zero_intermediate=True):
-        self._gemm2_exe, self._reduce_exe = gemm2_exe, reduce_exe
+        self._gemm2_exe = gemm2_exe
         self._topk, self._model_dim = int(topk), int(model_dim)
         self._out_dtype_str = out_dtype_str
         self._use_mask = bool(use_mask)
@@ -245,22 +258,20 @@ class _MoeGemm2ReduceWrapper:
         if self._use_mask and valid_mask is None:
             raise ValueError("this reduce-mode stage 2 was compiled with a valid mask; pass valid_mask")
         y = device_ptr(arg_out.view(-1), "Y", tokens * self._model_dim, dtypes=(_RED_DT[self._out_dtype_str],))
-        mask = valid_mask.contiguous().view(-1) if self._use_mask else None
-        mk = device_ptr(mask, "valid_mask", tokens * self._topk, elem_bytes=1) if self._use_mask else 0
         lib = _lib.load()
         kinds = (_lib.FLYGEMM_IN[g.in_dtype], _lib.FLYGEMM_OUT[_OUT[g.out_dtype][0]])
         zero = int(self._zero_intermediate and not self._use_mask)
         nbytes = lib.flygemm_moe_gemm2_reduce_scratch(tokens, self._topk, self._model_dim, zero)
-        rows = torch.empty(nbytes, dtype=torch.uint8, device=arg_out.device)
+        # The rows, and a copy of the mask, belong to the stream that uses them: the allocator hands a
+        # block out again in the order of its own stream only, and a copy queued on another stream
+        # may come after the kernels that read it.
+        with _on_stream(stream, h_stream, arg_out.device):
+            mask = valid_mask.contiguous().view(-1) if self._use_mask else None
+            rows = torch.empty(nbytes, dtype=torch.uint8, device=arg_out.device)
+        mk = device_ptr(mask, "valid_mask", tokens * self._topk, elem_bytes=1) if self._use_mask else 0
         rc = lib.flygemm_moe_gemm2_reduce(y, rows.data_ptr(), nbytes, *ptrs, *sizes, *kinds, int(g.doweight),
                                           int(g.blockscale), g.group_size, mk, zero, h_stream)
         _lib.check(rc, "flygemm_moe_gemm2_reduce")
-        if h_stream != torch.cuda.current_stream(arg_out.device).cuda_stream:
-            # the allocator hands memory out again in the order of the stream it came from
-            other = stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.ExternalStream(h_stream, arg_out.device)
-            rows.record_stream(other)
-            if mask is not None:
-                mask.record_stream(other)
 
     @property
     def mode(self) -> str:

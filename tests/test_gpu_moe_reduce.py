@@ -73,3 +73,54 @@ def test_other_stream(gpu):
     s2(got, *args, stream=side.cuda_stream)
     side.synchronize()
     assert torch.equal(got, want)
+
+
+def _stage2(topk, dim, **kw):
+    return compile_moe_gemm2_ex(model_dim=dim, inter_dim=256, experts=24, topk=topk, tile_m=32, tile_n=128, tile_k=128,
+                                doweight_stage2=True, in_dtype="fp8", out_dtype="f16", mode=MoeGemm2Mode.REDUCE, **kw)
+
+
+def _busy(big):
+    """Some twenty milliseconds of work on the current stream: far more than one layer takes."""
+    for _ in range(60):
+        big[1].copy_(big[0])
+
+
+@pytest.mark.parametrize("as_handle", [False, True])
+def test_other_stream_with_work_queued_on_the_current_one(gpu, as_handle):
+    """While the current stream still has work to do on a block that was handed back to the allocator,
+    a call for another stream neither takes that block for its rows nor reads a mask that the
+    current stream has yet to copy."""
+    tokens, topk, dim = 1025, 8, 1024
+    p, meta, blocks = _problem(tokens, topk, dim, 256, 24, 32, 11, gpu)
+    args = _args(p, meta, tokens, dim, 256, blocks)
+    want, want_m, got = (torch.empty(tokens * dim, dtype=torch.float16, device=gpu) for _ in range(3))
+    mask = (torch.rand(topk, tokens, device=gpu) < 0.5).to(torch.int8).t()     # not contiguous
+    kept = p["topk_ids"] < 11
+    mask &= kept                                                               # routes that have a row
+    plain, masked = _stage2(topk, dim), _stage2(topk, dim, valid_mask=mask)
+    plain(want, *args)
+    masked(want_m, *args, valid_mask=mask)
+    # a block of every size class that the rows (and the mask behind them) can come from
+    nbytes = [(tokens * topk * dim * 2 + 255) // 256 * 256 + m for m in (0, (tokens * topk + 255) // 256 * 256)]
+    after = [torch.empty(n, dtype=torch.uint8, device=gpu) for n in nbytes]
+    big = torch.zeros(2, 2 ** 30, dtype=torch.uint8, device=gpu)
+    side = torch.cuda.Stream()
+    stream = side.cuda_stream if as_handle else side
+    torch.cuda.synchronize()
+    for fn, kw, ref in ((plain, {}, want), (masked, dict(valid_mask=mask), want_m)):
+        fn(got, *args, stream=stream, **kw)     # (memory of the side stream's own, so that nothing waits below)
+        torch.cuda.synchronize()
+        got.zero_()
+        torch.cuda.synchronize()
+        held = [torch.full((n,), 7, dtype=torch.uint8, device=gpu) for n in nbytes]
+        _busy(big)
+        for a, h in zip(after, held):
+            a.copy_(h)
+        del held, h
+        fn(got, *args, stream=stream, **kw)
+        side.synchronize()
+        assert not torch.cuda.current_stream().query()      # the side call overtook the queued work
+        assert torch.equal(got, ref)
+        torch.cuda.synchronize()
+        assert all(bool((a == 7).all()) for a in after)
