@@ -68,8 +68,6 @@ MoeKernel moe_stage1_kernel(int kind, int tm, int r, int tn, bool bs) {
       default: return MoeKernel{nullptr, 0};
     }
   }
-  if (moe_stream_stage1(1, kind, bs))
-    return r * tm == 128 && tn == 64 ? moe_stage1_stream_kernel(kind, tm, false, false) : MoeKernel{nullptr, 0};
   return kind == KIND_W4A16 ? moe_stage1_tile<KIND_W4A16, false>(tm, r, tn) : MoeKernel{nullptr, 0};
 }
 
@@ -94,34 +92,25 @@ bool moe_large_experts(int kind, int inter, long routes, long experts) {
                            : (inter >= 1024 && routes >= 512L * experts) || (inter >= 4096 && routes >= 256L * experts);
 }
 
-// Tile of a call: runs of R routing blocks per workgroup and tile_n output columns (the
-// caller's tile_n, already validated, is a hint).  atomics: a stage-2 call that accumulates
-// (per-route-row calls take the stream kernel's tiles where it applies).
+// Tile of a call before the stream kernels' and the mid-sized routings' rules (moe_choose): runs of R
+// routing blocks per workgroup and tile_n output columns (the caller's tile_n, already validated,
+// is a hint).  atomics: a stage-2 call that accumulates.
 int moe_tiles(int stage, int tokens, int N, int K, int experts, int topk, int tile_m, int tile_n, int kind, bool bs,
               bool atomics, const char* what, int* r_out, int* tn_out, bool wgroup = false) {
   const long routes = (long)tokens * topk;
   const int inter = stage == 1 ? N : K;
-  // Blockscale on large experts (inter_dim of at least 1024): runs of 256 rows, 128 columns in
-  // stage 2 (16- and 32-row blocks from 128 routes per expert, 64-row blocks from 512) and 64 in
-  // stage 1 (16-row blocks only).  Graph-timed, DS-V3 prefill dims (7168 x 2048, 256 experts,
-  // top-8), single-block tiles against runs (µs): 16-row blocks, 16384 tokens stage 1 15736 ->
-  // 13737, stage 2 17192 -> 6105; 4096 tokens 4868 -> 4067 / 4495 -> 2036; 32-row blocks stage 2
-  // 8812 -> 5908 at 16384 tokens, 2453 -> 2032 at 4096, slower at 2048 (1386 -> 1713); 64-row
-  // blocks stage 2 7054 -> 5748 at 16384 tokens, level at 4096 (2032 / 2012); stage 1 slower on
-  // runs for 32- and 64-row blocks (9239 -> 12862), as is inter_dim 256 (8192 tokens, 16-row
-  // blocks, stage 2 909 -> 1196).
-  if (bs && inter >= 1024) {
-    if (stage == 2 && N % 128 == 0 &&
-        (tile_m == 64 ? routes >= 512L * experts : routes >= 128L * experts)) {
-      *r_out = 256 / tile_m;
-      *tn_out = 128;
-      return 0;
-    }
-    if (stage == 1 && tile_m == 16 && routes >= 128L * experts && N % 64 == 0) {
-      *r_out = 16;
-      *tn_out = 64;
-      return 0;
-    }
+  // Blockscale stage 2 on large experts (inter_dim of at least 1024): runs of 256 rows, 128 columns
+  // (16- and 32-row blocks from 128 routes per expert, 64-row blocks from 512).  Graph-timed, DS-V3
+  // prefill dims (7168 x 2048, 256 experts, top-8), single-block tiles against runs (µs): 16-row
+  // blocks, 16384 tokens 17192 -> 6105, 4096 tokens 4495 -> 2036; 32-row blocks 8812 -> 5908 at 16384
+  // tokens, 2453 -> 2032 at 4096, slower at 2048 (1386 -> 1713); 64-row blocks 7054 -> 5748 at 16384
+  // tokens, level at 4096 (2032 / 2012); slower at inter_dim 256 (8192 tokens, 16-row blocks 909 ->
+  // 1196).
+  if (bs && inter >= 1024 && stage == 2 && N % 128 == 0 &&
+      (tile_m == 64 ? routes >= 512L * experts : routes >= 128L * experts)) {
+    *r_out = 256 / tile_m;
+    *tn_out = 128;
+    return 0;
   }
   // Large experts (fp8, int8, bf16, fp16, int4; inter_dim of at least 1024, at least 512 routes per
   // expert on average; stage 1 with model_dim of at least 4096): runs of 256 rows (four 64-row,
@@ -272,17 +261,17 @@ bool moe_stage1_streams(int kind, bool bs, bool gs, int tile_m, int kb, long rou
 //   * W4A16 and blockscale (single blocks in moe_tiles) from 48 routes: blockscale 4096 x 1536 at 125
 //     routes, 16- / 32-row blocks 288 / 250 against 183 / 181, W4A16 4096 x 14336 at 75 routes, 16-row
 //     blocks 351 against 210; at 31 routes and fewer slower.
-bool moe_stage2_mid(int kind, bool bs, bool rows, int tile_m, int r, int kb, int n, long routes, long experts,
+void moe_stage2_mid(int kind, bool bs, bool rows, int tile_m, int r, int kb, int n, long routes, long experts,
                     int* r_out, int* tn_out) {
-  if (n % 128 != 0) return false;
+  if (n % 128 != 0) return;
   // moe_tiles' 256-row runs of large experts stay; 16-row blocks have runs from 32 routes per expert
   const bool runs16 = !bs && kind != KIND_W4A16 && tile_m == 16;
   const int inter = moe_a_16bit(kind) ? kb / 2 : kb;
-  if (r > 1 && !(runs16 && !moe_large_experts(kind, inter, routes, experts))) return false;
+  if (r > 1 && !(runs16 && !moe_large_experts(kind, inter, routes, experts))) return;
   const bool deep = kb >= 1024;
   const long from = bs || kind == KIND_W4A16 ? 48 : 32;
-  if (routes < from * experts || (!deep && !(runs16 && !rows))) return false;
-  if (tile_m == 64 && (rows || routes < 48 * experts)) return false;
+  if (routes < from * experts || (!deep && !(runs16 && !rows))) return;
+  if (tile_m == 64 && (rows || routes < 48 * experts)) return;
   const bool narrow = !deep && routes < 64 * experts;
   *tn_out = narrow ? 64 : 128;
   if (tile_m == 16)
@@ -291,7 +280,64 @@ bool moe_stage2_mid(int kind, bool bs, bool rows, int tile_m, int r, int kb, int
     *r_out = !rows || (routes >= 128 * experts && kind != KIND_INT4) ? 2 : 1;
   else
     *r_out = 1;
-  return true;
+}
+
+// What a call runs: a kernel family, R routing blocks per run and tile_n output columns.
+enum class MoePath { kTile, kStream1, kStream2, kStream2Single };
+struct MoeChoice {
+  MoePath path;
+  int r, tile_n;
+};
+
+// The choice for a call, the only one: the launchers and flygemm_moe_select_tile take it from here.
+// rows: a stage-2 call that writes per-route rows.
+int moe_choose(int stage, int tokens, int N, int K, int experts, int topk, int tile_m, int tile_n, int kind, bool bs,
+               bool rows, bool wgroup, const char* what, MoeChoice* c) {
+  const long routes = (long)tokens * topk;
+  const long kb = moe_a_16bit(kind) ? 2L * K : (long)K;   // activation bytes per row
+  c->path = MoePath::kTile;
+  if (int rc = moe_tiles(stage, tokens, N, K, experts, topk, tile_m, tile_n, kind, bs, stage == 2 && !rows, what, &c->r,
+                         &c->tile_n, wgroup))
+    return rc;
+  if (stage == 1) {
+    if (moe_stage1_streams(kind, bs, wgroup, tile_m, (int)kb, routes, experts)) {
+      *c = MoeChoice{MoePath::kStream1, (kind == KIND_W4A16 ? 64 : 128) / tile_m, 64};
+    } else if (moe_stream_stage1(stage, kind, bs) && c->r * tile_m == 128) {
+      c->path = MoePath::kStream1;
+    }
+    return 0;
+  }
+  // Stage 2 per-route rows (the reduce mode's GEMM) of 1-byte and 16-bit weights with inter_dim
+  // of 1, 2 or 4 128-byte K steps: the stream kernel (moe_stream.h), 64-column tiles, A resident,
+  // the next tile's weights loaded before this tile's stores.  With 1 to 32 routes per expert on
+  // average it runs single routing blocks (32 rows for 16-row blocks), each workgroup walking
+  // about 64 KB of weights (four 64-column tiles of fp8 at inter_dim 256, two of bf16); with a
+  // full 128-row run per expert on average (and for 16-row blocks from 32 routes per expert,
+  // wherever the kernel above takes 256-row runs) runs of 128 rows.  Graph-timed, bit-equal,
+  // reduce mode (GEMM + reduction), fp8, inter_dim 256, model_dim 7168: DS-TP8 decode dims (256
+  // experts, 32-row blocks) 32 / 128 / 256 / 512 tokens 49.0 / 98.5 / 106.7 / 117.4 us against
+  // 59.0 / 117.3 / 123.6 / 124.5 (single-block kernel above), 8 tokens level (20 us); bf16 2
+  // tiles per workgroup, 9-16% faster from 32 tokens; DS-TP8 prefill dims (128 experts) 128 / 512
+  // tokens 42.3 / 60.1 against 46.7 / 80.5 (16-row blocks, the latter against 128-row runs),
+  // 43.1 / 59.4 against 51.3 / 61.6 (64-row blocks); at 64 routes per expert (1024 tokens) single
+  // blocks were 3-6% slower for 16- and 64-row blocks, and 128-row runs win from 128 (64-row
+  // blocks 2048 / 4096 / 8192 tokens 146 / 246 / 438 us against 164 / 279 / 586 for the kernel
+  // above).  Fewer routes than experts (8 tokens top-8 of 256): the kernel above.
+  const long nk = kb / 128;
+  if (rows && !bs && kind != KIND_W4A16 && (nk == 1 || nk == 2 || nk == 4) && routes >= experts) {
+    const bool single = routes <= 32L * experts;
+    // (int4 weights, half the bytes per tile: 128-row runs from 256 routes per expert for 32- and
+    // 64-row blocks -- DS-TP8 prefill 4096 / 8192 tokens 232 / 443 us against 266 / 566 for the
+    // kernel above, at 2048 149 against 128)
+    const long runs_from = kind == KIND_INT4 ? 256L : 128L;
+    if (single || routes >= runs_from * experts || (tile_m == 16 && routes >= 32L * experts)) {
+      *c = single ? MoeChoice{MoePath::kStream2Single, tile_m == 16 ? 2 : 1, 64}
+                  : MoeChoice{MoePath::kStream2, 128 / tile_m, 64};
+      return 0;
+    }
+  }
+  moe_stage2_mid(kind, bs, rows, tile_m, c->r, (int)kb, N, routes, experts, &c->r, &c->tile_n);
+  return 0;
 }
 
 // in_dtype -> kernel kind (and whether stage-1 activations come per route); -1 if unknown
@@ -347,10 +393,12 @@ int moe_plan(int stage, void* out, const void* a, const void* w, const float* sa
   if (group_size > 0 && (kind != KIND_W4A16 || group_size != 32))
     return fail(hipErrorInvalidValue, "%s: group_size=%d: group scales are for int4_bf16 with group_size 32", what,
                 group_size);
-  int R = 1;
-  if (int rc = moe_tiles(stage, tokens, N, K, experts, topk, tile_m, tile_n, kind, bs, stage == 2 && accumulate != 0,
-                         what, &R, &tile_n, group_size > 0))
+  const bool rows = stage == 2 && !accumulate;
+  MoeChoice c;
+  if (int rc = moe_choose(stage, tokens, N, K, experts, topk, tile_m, tile_n, kind, bs, rows, group_size > 0, what, &c))
     return rc;
+  const int R = c.r;
+  tile_n = c.tile_n;
   const bool is16 = moe_a_16bit(kind);      // 2-byte activations (bf16, fp16, W4A16)
   const long kb = is16 ? 2L * K : (long)K;  // activation bytes per row
   if (kb % 128 != 0)
@@ -361,7 +409,6 @@ int moe_plan(int stage, void* out, const void* a, const void* w, const float* sa
   if (a_rows * kb >= (1L << 31) || w_rows * wb >= (1L << 31))
     return fail(hipErrorInvalidValue, "%s: activation or per-expert weight above 2^31 bytes", what);
   int mout;
-  const bool rows = stage == 2 && !accumulate;
   if (out_dtype == FLYGEMM_OUT_FP16) mout = rows ? MOE_OUT_F16_ROWS : MOE_OUT_F16;
   else if (out_dtype == FLYGEMM_OUT_BF16) mout = rows ? MOE_OUT_BF16_ROWS : MOE_OUT_BF16;
   else if (out_dtype == FLYGEMM_OUT_F32 && stage == 2 && accumulate) mout = MOE_OUT_F32;
@@ -381,55 +428,17 @@ int moe_plan(int stage, void* out, const void* a, const void* w, const float* sa
   if (bs && (2L * N) % (stage == 1 ? 128 : 256) != 0)
     return fail(hipErrorInvalidValue, "%s: %s=%d must be a multiple of 128 (weight scale blocks)", what,
                 stage == 1 ? "2*inter_dim" : "model_dim", stage == 1 ? 2 * N : N);
-  MoeKernel k = stage == 1 ? moe_stage1_kernel(kind, tile_m, R, tile_n, bs)
-                           : moe_stage2_kernel(kind, tile_m, R, tile_n, mout == MOE_OUT_F32, bs);
-  // Stage 2 per-route rows (the reduce mode's GEMM) of 1-byte and 16-bit weights with inter_dim
-  // of 1, 2 or 4 128-byte K steps: the stream kernel (moe_stream.h), 64-column tiles, A resident,
-  // the next tile's weights loaded before this tile's stores.  With 1 to 32 routes per expert on
-  // average it runs single routing blocks (32 rows for 16-row blocks), each workgroup walking
-  // about 64 KB of weights (four 64-column tiles of fp8 at inter_dim 256, two of bf16); with a
-  // full 128-row run per expert on average (and for 16-row blocks from 32 routes per expert,
-  // wherever the kernel above takes 256-row runs) runs of 128 rows.  Graph-timed, bit-equal,
-  // reduce mode (GEMM + reduction), fp8, inter_dim 256, model_dim 7168: DS-TP8 decode dims (256
-  // experts, 32-row blocks) 32 / 128 / 256 / 512 tokens 49.0 / 98.5 / 106.7 / 117.4 us against
-  // 59.0 / 117.3 / 123.6 / 124.5 (single-block kernel above), 8 tokens level (20 us); bf16 2
-  // tiles per workgroup, 9-16% faster from 32 tokens; DS-TP8 prefill dims (128 experts) 128 / 512
-  // tokens 42.3 / 60.1 against 46.7 / 80.5 (16-row blocks, the latter against 128-row runs),
-  // 43.1 / 59.4 against 51.3 / 61.6 (64-row blocks); at 64 routes per expert (1024 tokens) single
-  // blocks were 3-6% slower for 16- and 64-row blocks, and 128-row runs win from 128 (64-row
-  // blocks 2048 / 4096 / 8192 tokens 146 / 246 / 438 us against 164 / 279 / 586 for the kernel
-  // above).  Fewer routes than experts (8 tokens top-8 of 256): the kernel above.
-  bool stream2 = false, single2 = false;
-  const long routes_all = (long)tokens * topk;
-  if (stage == 2 && rows && !bs && kb <= 512 && routes_all >= experts) {
-    single2 = routes_all <= 32L * experts;
-    // (int4 weights, half the bytes per tile: 128-row runs from 256 routes per expert for 32- and
-    // 64-row blocks -- DS-TP8 prefill 4096 / 8192 tokens 232 / 443 us against 266 / 566 for the
-    // kernel above, at 2048 149 against 128)
-    const long runs_from = kind == KIND_INT4 ? 256L : 128L;
-    if (single2 || routes_all >= runs_from * experts || (tile_m == 16 && routes_all >= 32L * experts)) {
-      const MoeKernel k2 = moe_stage2_stream_kernel(kind, tile_m, (int)(kb / 128), single2);
-      if (k2.fn) {
-        k = k2;
-        R = single2 ? (tile_m == 16 ? 2 : 1) : 128 / tile_m;
-        tile_n = 64;
-        stream2 = true;
-      }
-    }
-  }
-  const bool stream1 = stage == 1 && moe_stage1_streams(kind, bs, group_size > 0, tile_m, (int)kb, routes_all, experts);
-  if (stream1) {
-    k = moe_stage1_stream_kernel(kind, tile_m, bs, group_size > 0);
-    R = (kind == KIND_W4A16 ? 64 : 128) / tile_m;
-    tile_n = 64;
-  }
-  if (stage == 2 && !stream2 &&
-      moe_stage2_mid(kind, bs, rows, tile_m, R, (int)kb, N, routes_all, experts, &R, &tile_n))
-    k = moe_stage2_kernel(kind, tile_m, R, tile_n, mout == MOE_OUT_F32, bs);
+  const bool single2 = c.path == MoePath::kStream2Single, stream2 = single2 || c.path == MoePath::kStream2;
+  const bool stream1 = c.path == MoePath::kStream1;
+  const MoeKernel k = stream1      ? moe_stage1_stream_kernel(kind, tile_m, bs, group_size > 0)
+                      : stream2    ? moe_stage2_stream_kernel(kind, tile_m, (int)(kb / 128), single2)
+                      : stage == 1 ? moe_stage1_kernel(kind, tile_m, R, tile_n, bs)
+                                   : moe_stage2_kernel(kind, tile_m, R, tile_n, mout == MOE_OUT_F32, bs);
   if (!k.fn) return fail(hipErrorInvalidValue, "%s: no kernel for tile %dx%d (runs of %d)", what, tile_m, tile_n, R);
 
   // column ranges per run: about 1024 workgroups in all (the stream kernel: one column tile each)
   const long ntn = N / tile_n;
+  const long routes_all = (long)tokens * topk;
   const long runs = est_runs(tokens, topk, experts, tile_m, R);
   long nsplit = (1024 + runs - 1) / runs;
   nsplit = nsplit < 1 ? 1 : (nsplit > ntn ? ntn : nsplit);
@@ -451,7 +460,7 @@ int moe_plan(int stage, void* out, const void* a, const void* w, const float* sa
   // single blocks: about 64 KB of weights per workgroup (DS-TP8 decode dims, 32 tokens: fp8 28
   // ranges of four tiles 49.0 us, 4 ranges 52.6, 56 ranges 52.6; bf16 56 ranges of two 105.8
   // against 107.9 for 28)
-  if (stream2 && single2) {
+  if (single2) {
     const long per = std::max(1L, 65536L / ((long)tile_n * kb));
     nsplit = (ntn + per - 1) / per;
   }
@@ -682,12 +691,11 @@ int flygemm_moe_select_tile(int32_t stage, int32_t tokens, int32_t n, int32_t k,
   bool token_slot = false;
   const int kind = moe_kind(in_dtype, stage, &token_slot);
   if (kind < 0) return fail(hipErrorInvalidValue, "%s: in_dtype %d not supported", what, in_dtype);
-  int r = 1, tn = 0;
-  if (int rc = moe_tiles(stage, tokens, n, k, experts, topk, tile_m, tile_n, kind, blockscale != 0, stage == 2, what, &r,
-                         &tn))
+  MoeChoice c;
+  if (int rc = moe_choose(stage, tokens, n, k, experts, topk, tile_m, tile_n, kind, blockscale != 0, false, false, what, &c))
     return rc;
-  *runs = r;
-  *tile_n_out = tn;
+  *runs = c.r;
+  *tile_n_out = c.tile_n;
   return 0;
 }
 

@@ -207,17 +207,15 @@ int flygemm_moe_blockscale_gemm2(void* out, const void* a2, const void* w, const
                                  int32_t tile_n, int32_t scale_block_k, int32_t out_dtype, int32_t doweight_stage2,
                                  int32_t accumulate, void* stream);
 
-/* The MoE launchers' tile choice for a call with these sizes (they treat tile_n as a hint):
- * *runs = routing blocks per workgroup (1: single-block tiles; more: runs of 128 rows in stage
- * 1, 256 in stage 2, and 256 in stage 1 of routings with large experts, blockscale included) and *tile_n_out =
- * output columns per tile.  Stage 2 values are those of accumulating calls; per-route-row calls
- * (accumulate = 0) of 1-byte, int4 (int8 activations) and 16-bit weights with inter_dim of 1, 2
- * or 4 128-byte K steps run 64-column tiles instead: single routing blocks (two for tile_m 16)
- * with 1 to 32 routes per expert on average, 128-row runs from 128 routes per expert (int4: 256;
- * from 32 for tile_m 16).  Stage 1 of W4A16 with a model_dim of whole 256-element steps and of
- * blockscale leaves this choice for the stream kernel's runs (64 and 128 rows, 64 columns) at the
- * routes per expert that csrc/moe.hip names, and stage 2 of routings between decode and large
- * experts for runs of 32 and 64 rows.  n is the GEMM's output width and k its depth (stage 1: inter_dim and
+/* The MoE launchers' tile choice for a call with these sizes (they treat tile_n as a hint), from
+ * the function that they call themselves: *runs = routing blocks per workgroup (1: single-block
+ * tiles; more: runs of 32, 64, 128 or 256 rows) and *tile_n_out = output columns per tile.  The
+ * choice is that of a stage-2 call that accumulates and of W4A16 with per-row scales; calls that
+ * write per-route rows (accumulate = 0) or take group scales can differ: rows of 1-byte, int4 (int8
+ * activations) and 16-bit weights with inter_dim of 1, 2 or 4 128-byte K steps run 64-column tiles,
+ * single routing blocks (two for tile_m 16) with 1 to 32 routes per expert on average, 128-row runs
+ * from 128 routes per expert (int4: 256; from 32 for tile_m 16).  csrc/moe.hip has the rules and their
+ * figures.  n is the GEMM's output width and k its depth (stage 1: inter_dim and
  * model_dim; stage 2: model_dim and inter_dim); in_dtype as for flygemm_moe_gemm1/2; blockscale
  * != 0 for the blockscale MoE.  Validates like the launchers; touches no device.  Counterpart of
  * the reference's compile-time tile arguments (kernels/moe_gemm_2stage.py:93-121), for tests and

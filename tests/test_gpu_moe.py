@@ -588,12 +588,12 @@ def run_bs_stage2(p, dev, out_dtype="f16", doweight=True, mode="atomic"):
 def test_blockscale_run_tiles(gpu, tile_m):
     """Blockscale MoE with large experts (1100 tokens top-2 of 4 experts, model_dim 1024,
     inter_dim 1024: 550 routes per expert), checked through flygemm_moe_select_tile first: stage
-    2 on runs of 256 rows x 128 columns (atomics and per-route rows), stage 1 on runs of 256 rows
-    x 64 columns for 16-row blocks (single-block tiles for 32- and 64-row ones); some runs partial."""
+    2 on runs of 256 rows x 128 columns (atomics and per-route rows), stage 1 on the stream
+    kernel's runs of 128 rows; some runs partial."""
     w = W.moe_custom(1100, 1024, 1024, 4, 2, tile_m, 128, 256, "fp8_block", seed=41)
     R = 256 // tile_m
     assert _chosen_tile(2, w, "fp8", 1) == (R, 128)
-    assert _chosen_tile(1, w, "fp8", 1)[0] == (R if tile_m == 16 else 1)
+    assert _chosen_tile(1, w, "fp8", 1) == (128 // tile_m, 64)
     p = W.moe_problem(w, gpu)
     counts = np.bincount(_np(p["topk_ids"]).ravel(), minlength=w.experts)
     assert ((counts + tile_m - 1) // tile_m % R != 0).any(), counts
@@ -713,8 +713,10 @@ def test_new_kinds_every_tile(gpu, kind, group, tile_m, tile_n):
 @pytest.mark.parametrize("tile_m", [16, 64])
 def test_new_kinds_runs_of_blocks(gpu, kind, tile_m):
     """Experts with many routing blocks: stage 1 on the stream kernel's 128-row runs, stage 2 on
-    the 8-wave run tiles (16-row blocks) or single-block tiles."""
+    runs of 64 rows (16-row blocks) or single-block tiles."""
     w = W.moe_custom(600, 512, 256, 5, 2, tile_m, 128, 256, kind, seed=tile_m * 3)
+    assert _chosen_tile(1, w, kind) == (128 // tile_m, 64)
+    assert _chosen_tile(2, w, kind) == ((4, 128) if tile_m == 16 else (1, 64))
     p = W.moe_problem(w, gpu)
     rows = np.unique(np.r_[np.arange(0, 600, 7), 599])
     _say(f"runs {kind} tile_m {tile_m}")
@@ -787,15 +789,14 @@ WIDE_KINDS = [("fp8", -1), ("int8", -1), ("bf16", -1), ("fp16", -1), ("int4", -1
 @pytest.mark.parametrize("kind,group", WIDE_KINDS, ids=[k if g < 0 else f"{k}-g{g}" for k, g in WIDE_KINDS])
 def test_single_block_wide_tiles(gpu, kind, group):
     """Routings with about one block per expert (top-4 of 64 experts, D = 512, I = 1024, tile_m
-    32, tile_n hints 256), checked through flygemm_moe_select_tile first: 512 tokens -> stage 1
-    of W4A16 on the 128-column single-block kernel, stage 2 with atomics on 64-column tiles (32
-    routes per expert); 160 tokens -> W4A16 stage 1 on 64 columns, stage 2 with atomics on the
-    128-column kernel (10 routes per expert).  The other kinds' stage 1 runs the stream kernel.
-    Stage 2 in atomic and reduce modes."""
-    for tokens, s1, s2 in ((512, (1, 128), (1, 64)), (160, (1, 64), (1, 128))):
+    32, tile_n hints 256), checked through flygemm_moe_select_tile first: 512 tokens -> stage 2 with
+    atomics on runs of 64 rows (W4A16: 64-column tiles; 32 routes per expert), 160 tokens -> on the 128-column kernel (10
+    routes per expert).  Stage 1 runs the stream kernel (W4A16 on its LDS-staged tiles:
+    test_w4a16_stage1_lds_tiles of test_gpu_moe_mid.py).  Stage 2 in atomic and reduce modes."""
+    for tokens, s2 in ((512, (1, 64) if kind == "int4_bf16" else (2, 128)), (160, (1, 128))):
         w = W.moe_custom(tokens, 512, 1024, 64, 4, 32, 256, 256, kind, seed=11 + tokens)
-        # (stage 1 of the other kinds: the stream kernel's 128-row runs of 64 columns)
-        assert _chosen_tile(1, w, kind) == (s1 if kind == "int4_bf16" else (4, 64))
+        # the stream kernel's 64- and 128-row runs of 64 columns
+        assert _chosen_tile(1, w, kind) == ((2, 64) if kind == "int4_bf16" else (4, 64))
         assert _chosen_tile(2, w, kind) == s2
         p = W.moe_problem(w, gpu, group_size=group)
         p["group_size"] = group
@@ -823,9 +824,10 @@ def test_single_block_wide_tiles(gpu, kind, group):
 
 
 def test_single_block_wide_tiles_blockscale(gpu):
-    """The same routings through the blockscale MoE: 512 tokens -> stage 1 single-block
-    128-column tiles, stage 2 64-column ones; 160 tokens -> 64 and 128 columns."""
-    for tokens, s1, s2 in ((512, (1, 128), (1, 64)), (160, (1, 64), (1, 128))):
+    """The same routings through the blockscale MoE: 512 tokens -> stage 1 on the stream kernel,
+    stage 2 on 64-column tiles; 320 and 160 tokens -> stage 1 on single-block tiles of 128 and 64
+    columns, stage 2 on 64 and 128."""
+    for tokens, s1, s2 in ((512, (4, 64), (1, 64)), (320, (1, 128), (1, 64)), (160, (1, 64), (1, 128))):
         _wide_blockscale(gpu, tokens, s1, s2)
 
 
@@ -874,18 +876,27 @@ def test_large_expert_run_tiles(gpu, kind, tile_m):
 @pytest.mark.parametrize("tile_m", [64, 32])
 def test_large_expert_run_tiles_w4a16(gpu, tile_m):
     """W4A16 with per-row weight scales on large experts (1100 tokens top-2 of 4 experts,
-    model_dim 4096, inter_dim 1024): runs of 256 rows in both stages; with group scales the
-    single-block tiles stay.  A sample of tokens against the oracle."""
-    w = W.moe_custom(1100, 4096, 1024, 4, 2, tile_m, 128, 256, "int4_bf16", seed=43)
+    inter_dim 1024): stage 2 on runs of 256 rows (model_dim 4096); stage 1 on the stream kernel there,
+    and on runs of 256 rows where model_dim is no whole number of its steps (4160).  A sample of
+    tokens against the oracle."""
     R = 256 // tile_m
-    assert _chosen_tile(1, w, "int4_bf16") == (R, 128) and _chosen_tile(2, w, "int4_bf16") == (R, 256)
+    w = W.moe_custom(1100, 4160, 1024, 4, 2, tile_m, 128, 64, "int4_bf16", seed=43)
+    assert _chosen_tile(1, w, "int4_bf16") == (R, 128)
+    p = W.moe_problem(w, gpu, with_stage2_input=False)
+    rows = np.unique(np.r_[np.linspace(0, w.tokens - 1, 40).astype(int), w.tokens - 1])
+    _say(f"large-expert run tiles W4A16 tm{tile_m}, model_dim 4160")
+    o1 = run_stage1(p, gpu, "bf16", doweight=True)
+    torch.cuda.synchronize()
+    check_stage1(p, o1, True, rows, rows, what=f"W4A16 runs tm{tile_m} stage1")
+    w = W.moe_custom(1100, 4096, 1024, 4, 2, tile_m, 128, 256, "int4_bf16", seed=43)
+    assert _chosen_tile(1, w, "int4_bf16") == (64 // tile_m, 64) and _chosen_tile(2, w, "int4_bf16") == (R, 256)
     p = W.moe_problem(w, gpu)
     rows = np.unique(np.r_[np.linspace(0, w.tokens - 1, 40).astype(int), w.tokens - 1])
     _say(f"large-expert run tiles W4A16 tm{tile_m}")
     o1 = run_stage1(p, gpu, "bf16", doweight=True)
     o2 = run_stage2(p, gpu, "f32", doweight=True)
     torch.cuda.synchronize()
-    check_stage1(p, o1, True, rows, rows, what=f"W4A16 runs tm{tile_m} stage1")
+    check_stage1(p, o1, True, rows, rows, what=f"W4A16 large experts tm{tile_m} stage1")
     check_stage2(p, o2, True, rows, rows, what=f"W4A16 runs tm{tile_m} stage2")
 
 

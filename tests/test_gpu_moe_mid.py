@@ -24,6 +24,20 @@ def test_w4a16_stage1_stream(gpu, group, tile_m, tokens):
         M.check_stage1(p, out, K % 512 == 0, what=f"W4A16 g{group} tm{tile_m} t{tokens} K{K}")
 
 
+@pytest.mark.parametrize("group", [-1, 32])
+@pytest.mark.parametrize("tokens,tile", [(512, (1, 128)), (160, (1, 64))])
+def test_w4a16_stage1_lds_tiles(gpu, group, tokens, tile):
+    """Stage 1 of W4A16 where model_dim is no whole number of 256-element steps: single-block tiles of
+    128 columns from about three workgroups per CU, else of 64."""
+    w = W.moe_custom(tokens, 576, 1024, 64, 4, 32, 256, 64, "int4_bf16", seed=tokens)
+    assert M._chosen_tile(1, w, "int4_bf16") == tile
+    p = W.moe_problem(w, gpu, group_size=group, with_stage2_input=False)
+    # (group scales: against the oracle's truncation, and against the exact dequantization, an
+    # approximate bound, on the smaller routing)
+    M.check_stage1(p, M.run_stage1(p, gpu, "bf16", doweight=True), True, what=f"W4A16 g{group} LDS tiles t{tokens}",
+                   exact=tokens == 160)
+
+
 @pytest.mark.parametrize("tile_m", [16, 32, 64])
 @pytest.mark.parametrize("tokens", [67, 190, 700])
 def test_blockscale_stage1_stream(gpu, tile_m, tokens):

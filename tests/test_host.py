@@ -456,10 +456,10 @@ def test_moe_blockscale_validation():
 def test_moe_tile_choice_pinned():
     """flygemm_moe_select_tile gives the launchers' tile choice without a device: stage 1 of
     1-byte, 16-bit and W4A8 weights runs the stream kernel (runs of 128 rows, 64 columns) but
-    for large experts; W4A16 and blockscale stage 1 keep single-block tiles but blockscale's
-    large experts of 16-row blocks; stage 2 takes runs for
-    16-row blocks of prefill routings, 64 columns for decode-sized ones, wide single-block tiles
-    in between (the reachable kernel set the GPU tests cover), and the launchers' validation."""
+    for large experts, that of W4A16 (runs of 64 rows) and of blockscale with enough routes per
+    expert too, else LDS-staged tiles; stage 2 takes runs of 32, 64 and 256 rows, 64 columns for
+    decode-sized routings, wide single-block tiles in between (the reachable kernel set the GPU
+    tests cover), and the launchers' validation."""
     import ctypes
     lib = _lib.load()
 
@@ -478,22 +478,25 @@ def test_moe_tile_choice_pinned():
             for tm in (16, 32, 64):
                 assert sel(1, tokens, n, experts, topk, tm, 256, kind) == (128 // tm, 64), (kind, tokens, tm)
     # stage 2 (accumulating calls) on DS-TP8 prefill: 64-column single-block tiles for 32- and
-    # 64-row blocks (16+ routes per expert), runs of 256 rows and 256 columns for 16-row blocks
+    # 64-row blocks (16+ routes per expert), runs of 64 rows and 128 columns for 16-row blocks
     assert sel(2, 8192, 7168, 128, 8, 64, 256) == (1, 64)
     assert sel(2, 8192, 7168, 128, 8, 32, 256) == (1, 64)
     assert sel(2, 8192, 7168, 128, 8, 64, 128) == (1, 64)
     assert sel(2, 1024, 7168, 128, 8, 64, 256) == (1, 64)     # 64 routes per expert
     assert sel(2, 160, 7168, 128, 8, 64, 256) == (1, 128)     # 10 routes per expert
-    assert sel(2, 8192, 7168, 128, 8, 16, 256) == (16, 256)
-    assert sel(2, 8192, 7168, 128, 8, 16, 256, "int4") == (16, 256)
+    assert sel(2, 8192, 7168, 128, 8, 16, 256) == (4, 128)
+    assert sel(2, 8192, 7168, 128, 8, 16, 256, "int4") == (4, 128)
     # decode: 64-column single-block tiles whatever the caller asked
-    assert sel(1, 8, 256, 256, 8, 32, 256, "int4_bf16") == (1, 64)
+    assert sel(1, 8, 256, 256, 8, 32, 256, "int4_bf16", k=7232) == (1, 64)
+    assert sel(1, 8, 256, 256, 8, 32, 256, "int4_bf16") == (2, 64)      # whole 256-element steps: 64-row runs
     assert sel(2, 8, 7168, 256, 8, 32, 256) == (1, 64)
-    # in between: stage 1 of W4A16 and blockscale 128 columns from about three workgroups per CU
-    # (runs x inter_dim / 128 >= 768), else 64; stage 2 never keeps 256 single-block columns
-    assert sel(1, 160, 1024, 64, 4, 32, 256, "int4_bf16") == (1, 64)      # 84 runs x 8 = 672
-    assert sel(1, 512, 1024, 64, 4, 32, 256, "int4_bf16") == (1, 128)     # 128 runs x 8
-    assert sel(1, 512, 1024, 64, 4, 32, 128, "fp8", 1) == (1, 128)
+    # in between: stage 1 of W4A16 and blockscale off the stream kernel 128 columns from about three
+    # workgroups per CU (runs x inter_dim / 128 >= 768), else 64; stage 2 never keeps 256 single-block columns
+    assert sel(1, 160, 1024, 64, 4, 32, 256, "int4_bf16", k=7232) == (1, 64)      # 84 runs x 8 = 672
+    assert sel(1, 512, 1024, 64, 4, 32, 256, "int4_bf16", k=7232) == (1, 128)     # 128 runs x 8
+    assert sel(1, 512, 1024, 64, 4, 32, 256, "int4_bf16") == (2, 64)
+    assert sel(1, 320, 1024, 64, 4, 32, 128, "fp8", 1) == (1, 128)
+    assert sel(1, 512, 1024, 64, 4, 32, 128, "fp8", 1) == (4, 64)
     assert sel(1, 160, 1024, 64, 4, 32, 256, "fp8", 1) == (1, 64)
     for kind in ("fp8", "int8", "bf16", "fp16", "int4", "int8smooth", "int4_bf16"):
         assert sel(2, 160, 512, 64, 4, 32, 256, kind) == (1, 128), kind
@@ -519,37 +522,75 @@ def test_moe_tile_choice_pinned():
         assert sel(1, 32768, 8192, 16, 4, 64, 128, kind, k=8192) == (4, 128), kind
         assert sel(2, 32768, 8192, 16, 4, 64, 256, kind, k=8192) == (4, 256), kind
     assert sel(2, 32768, 8192, 16, 4, 64, 256, "int4_bf16", k=8192) == (4, 256)    # W4A16, per-row scales
-    assert sel(1, 32768, 8192, 16, 4, 32, 128, "int4_bf16", k=8192) == (8, 128)
-    assert sel(1, 32768, 8192, 16, 4, 16, 128, "int4_bf16", k=8192)[0] == 1     # not for 16-row blocks
+    assert sel(1, 32768, 8192, 16, 4, 32, 128, "int4_bf16", k=8256) == (8, 128)
+    assert sel(1, 32768, 8192, 16, 4, 32, 128, "int4_bf16", k=8192) == (2, 64)  # the stream kernel
+    assert sel(1, 32768, 8192, 16, 4, 16, 128, "int4_bf16", k=8256)[0] == 1     # not for 16-row blocks
     assert sel(1, 32768, 8192, 16, 4, 64, 128, "int4", k=8192) == (4, 128)    # int4 from inter_dim 4096
     assert sel(2, 32768, 8192, 16, 4, 64, 256, "int4", k=8192) == (4, 256)
     assert sel(1, 32768, 2048, 16, 4, 64, 128, "int4", k=8192) == (2, 64)
     assert sel(2, 32768, 8192, 16, 4, 64, 256, "int4", k=2048)[0] == 1
     # blockscale on large experts (inter_dim >= 1024): stage 2 runs of 256 rows x 128 columns for
-    # 16-row blocks from 128 routes per expert and 64-row blocks from 512; stage 1 runs of 256 rows
-    # x 64 columns for 16-row blocks only
+    # 16-row blocks from 128 routes per expert and 64-row blocks from 512 (between: runs of 64 rows);
+    # stage 1 the stream kernel
     assert sel(2, 32768, 8192, 16, 4, 64, 256, "fp8", 1, k=8192) == (4, 128)
     assert sel(2, 16384, 7168, 256, 8, 16, 256, "fp8", 1, k=2048) == (16, 128)
     assert sel(2, 4096, 7168, 256, 8, 16, 256, "fp8", 1, k=2048) == (16, 128)      # 128 routes per expert
     assert sel(2, 4096, 7168, 256, 8, 64, 256, "fp8", 1, k=2048)[0] == 1           # 64-row blocks: 512
     assert sel(2, 4096, 7168, 256, 8, 32, 256, "fp8", 1, k=2048) == (8, 128)       # 32-row blocks: 128
-    assert sel(2, 2048, 7168, 256, 8, 32, 256, "fp8", 1, k=2048)[0] == 1
-    assert sel(1, 16384, 2048, 256, 8, 32, 256, "fp8", 1, k=7168)[0] == 1
-    assert sel(1, 16384, 2048, 256, 8, 16, 256, "fp8", 1, k=7168) == (16, 64)
-    assert sel(1, 16384, 2048, 256, 8, 64, 256, "fp8", 1, k=7168)[0] == 1
+    assert sel(2, 2048, 7168, 256, 8, 32, 256, "fp8", 1, k=2048) == (2, 128)
+    for tm in (16, 32, 64):
+        assert sel(1, 16384, 2048, 256, 8, tm, 256, "fp8", 1, k=7168) == (128 // tm, 64)
     assert sel(2, 8192, 7168, 256, 8, 16, 256, "fp8", 1, k=256)[0] == 1            # inter_dim 256
     assert lib.flygemm_moe_select_tile(1, 64, 256, 0, 4, 2, 64, 0, 0, 0, ctypes.byref(ctypes.c_int32()),
                                        ctypes.byref(ctypes.c_int32())) != 0   # k = 0
-    # blockscale (inter_dim 256) and W4A16 take no run tiles
+    # blockscale (inter_dim 256) and W4A16 take no run tiles in stage 2 there
     assert sel(2, 8192, 7168, 128, 8, 16, 256, "fp8", 1)[0] == 1
     assert sel(2, 8192, 7168, 128, 8, 16, 256, "int4_bf16")[0] == 1
-    assert sel(1, 8192, 256, 128, 8, 16, 256, "fp8", 1)[0] == 1
-    assert sel(1, 8192, 256, 128, 8, 16, 256, "int4_bf16")[0] == 1
+    assert sel(1, 8192, 256, 128, 8, 16, 256, "fp8", 1) == (8, 64)
+    assert sel(1, 8192, 256, 128, 8, 16, 256, "int4_bf16") == (4, 64)
+    assert sel(1, 8192, 256, 128, 8, 16, 256, "int4_bf16", k=7232)[0] == 1
     # validation
     assert sel(3, 16, 256, 4, 2, 16, 64) != 0 and b"stage" in lib.flygemm_last_error()
     assert sel(1, 16, 256, 4, 2, 48, 64) != 0 and b"tile_m" in lib.flygemm_last_error()
     assert sel(1, 16, 320, 4, 2, 16, 256) != 0 and b"tile_n" in lib.flygemm_last_error()
     assert sel(1, 16, 256, 4, 2, 16, 64, "fp4") != 0 and b"in_dtype" in lib.flygemm_last_error()
+
+
+def test_moe_tile_choice_reaches_built_kernels():
+    """Over a spread of sizes, every choice is a tile that the kernel tables hold for its kind: a call
+    with another one would be refused."""
+    import ctypes
+    import random
+    lib, rng = _lib.load(), random.Random(5)
+    r, tn = ctypes.c_int32(), ctypes.c_int32()
+    seen = set()
+    for _ in range(20000):
+        stage, tm = rng.choice((1, 2)), rng.choice((16, 32, 64))
+        kind, bs = rng.choice([(k, 0) for k in ("fp8", "int8", "int8smooth", "int4", "int4_bf16", "bf16", "fp16")] + [("fp8", 1)])
+        n, k = 128 * int(2 ** rng.uniform(0, 7)), 128 * int(2 ** rng.uniform(0, 7)) + rng.choice((0, 0, 64 if "16" in kind else 0))
+        experts = rng.choice((4, 17, 64, 256))
+        tokens = max(1, int(2 ** rng.uniform(0, 16) * experts / 64))
+        tile_n = rng.choice([t for t in (0, 64, 128, 256) if t == 0 or n % t == 0])
+        assert lib.flygemm_moe_select_tile(stage, tokens, n, k, experts, rng.choice((1, 2, 8)), tm, tile_n,
+                                           _lib.FLYGEMM_IN[kind], bs, ctypes.byref(r), ctypes.byref(tn)) == 0
+        w4, got = kind == "int4_bf16", (r.value, tn.value)
+        if stage == 1:
+            want = {((64 if w4 else 128) // tm, 64)}                            # the stream kernel
+            if w4 or bs:
+                want |= {(1, 64), (1, 128)}
+            if not bs and (not w4 or tm > 16):
+                want |= {(256 // tm, 128)}
+        else:
+            want = {(1, 64), (1, 128), (256 // tm, 128 if bs else 256)}
+            want |= {16: {(4, 128)}, 32: {(2, 128)}, 64: set()}[tm]
+            if tm == 16 and not (bs or w4):
+                want |= {(2, 64)}
+            if tm == 16 and w4:
+                want -= {(16, 256)}
+        assert got in want and n % got[1] == 0, (stage, kind, bs, tm, n, k, tokens, experts, got)
+        seen.add((stage, kind, bs, tm, *got))
+    # stages x (kinds and blockscale) x tile_m, most with three tiles and more
+    assert len(seen) > 120, len(seen)
 
 
 def test_compile_validates_on_first_call():
