@@ -224,22 +224,53 @@ int moe_tiles(int stage, int tokens, int N, int K, int experts, int topk, int ti
 
 // Stage 1 of W4A16 and of blockscale on the stream kernel (runs of 64 and 128 rows, 64 columns), in
 // place of moe_tiles' LDS-staged tiles.  Those re-read the weights for every 16 to 64 rows and have
-// one 128-byte K tile in flight, of which W4A16's share of the weights is 1 KB per 16 columns.
-// Graph-timed on MI355X (us, the LDS-staged choice against this kernel; blockscale bit-equal):
-//   W4A16, per-row scales: 7168 x 256, 128 experts, top-8: 4 / 256 / 2048 / 8192 tokens, 16-row
-//   blocks 53.3 / 108.5 / 530 / 1583 against 42.4 / 92.1 / 176 / 540, 64-row blocks 63.9 / 72.6 / 240 /
-//   711 against 41.6 / 60.9 / 172 / 521; 4096 x 14336, 8 experts, top-2: 1 / 32 / 600 / 3000 tokens,
-//   64-row blocks 43.3 / 161 / 474 / 1902 (runs of 256 rows) against 37.0 / 128 / 408 / 1669.  Its steps
-//   are four K tiles of A, so K must be a multiple of 256 elements.
-//   Group scales gain alike (6144 x 1024, 128 experts, 1000 tokens, 32-row blocks 760 against 454) but
-//   with fewer than 4 routes per expert (4096 x 2048, 17 experts, 4 tokens 66.5 against 70.2).
-//   Blockscale, 64-row blocks: 7168 x 256, 256 experts, 2 / 4 / 31 / 125 routes per expert 106 / 166 / 243
-//   / 368 against 128 / 145 / 194 / 283; 32-row: 4 / 8 / 31 / 125 routes 147 / 150 / 238 / 538 against 146 /
-//   150 / 198 / 296; 4096 x 1536, 64 experts, 16-row blocks, 8 / 16 / 31 / 62 / 250 / 750 routes 141 / 146 /
-//   217 / 361 / 766 / 1767 against 151 / 168 / 167 / 192 / 402 / 915.
-bool moe_stage1_streams(int kind, bool bs, bool gs, int tile_m, int kb, long routes, long experts) {
-  if (bs) return routes >= (tile_m == 64 ? 4 : 24) * experts;
-  return kind == KIND_W4A16 && kb % 512 == 0 && (!gs || routes >= 4 * experts);
+// one 128-byte K tile in flight, of which W4A16's share of the weights is 1 KB per 16 columns; the
+// stream kernel pays with rows of padding where experts have fewer rows than a run, and with fewer
+// workgroups (wg below; two share a CU).  Graph-timed on MI355X over ten sets of dims (model_dim 1024
+// to 8192, inter_dim 256 to 14336, 8 to 256 experts; us, the LDS-staged choice against this kernel;
+// blockscale bit-equal):
+//   W4A16, per-row and group scales (from 4 routes per expert; below they are level): 1.1-1.7x for
+//   64-row blocks throughout and for 16- and 32-row blocks from 24 routes per expert, up to 3x with
+//   16-row blocks (7168 x 256, 256 experts, 256 routes per expert), and level at worst on large
+//   experts, also where moe_tiles takes runs of 256 rows (8192 x 8192, 16 experts, 32-row blocks, 768 /
+//   1024 / 1536 routes 4114 / 5855 / 8189 against 4138 / 5437 / 8101).  With fewer routes and 16- or
+//   32-row blocks it also wins, but for model_dims of up to 4096 (16 steps) once the workgroups take a
+//   second round: 2048 x 768, 128 experts, 4 routes per expert, 16-row blocks 49.7 against 58.0;
+//   4096 x 2048, 17 experts, 8 routes 54.0 against 59.3; 4096 x 1536, 64 experts, 8 routes, 32-row
+//   blocks with group scales 128 against 147.  Its steps are four K tiles of A, so K must be a
+//   multiple of 256 elements.
+//   Blockscale.  Few workgroups lose whatever the routing: 1024 x 256, 8 experts, 24 to 384 routes per
+//   expert (36 to 128 workgroups), 16- / 32- / 64-row blocks 5.6-10.3 / 6.5-8.7 / 9.2-9.8 against
+//   10.5-12.8; at 1024 routes (288) 20.7 / 16.1 / 15.0 against 16.0 / 14.5 / 13.7.  16-row blocks from
+//   32 routes per expert and 384 workgroups (4096 x 512, 32 experts, 24 / 64 / 96 routes 27.1 / 57.3 /
+//   77.7 against 37.0 / 62.0 / 43.4; 7168 x 256, 128 experts, 24 / 32 / 128 routes 104 / 154 / 387
+//   against 120 / 126 / 162).  32-row blocks later, as their tiles re-read the weights half as often:
+//   from 64 routes (4096 x 512: 40 / 96 routes 26.6 / 46.4 against 37.1 / 39.6), with 896 workgroups from
+//   48, with 1536 from 24 (6144 x 1024, 128 experts, 24 routes 356 against 292; 7168 x 256, 256 experts,
+//   1344 workgroups, 40 routes 199 against 223).  64-row blocks: from 96 routes (4096 x 2048, 17 experts,
+//   64 / 96 routes 68.3 / 122 against 71.6 / 75.1); with 896 workgroups from 4 routes for model_dims
+//   above 6144 (7168 x 256, 256 experts, 8 routes 184 against 155), from 16 for 4096 (4096 x 1536, 64
+//   experts, 16 routes 165 against 141; 6144 x 1024, 8 routes 248 against 259), from 40 below
+//   (2048 x 768, 128 experts, 32 / 40 routes 79.2 / 108 against 90.8 / 88.1).
+bool moe_stage1_streams(int kind, bool bs, bool gs, int tile_m, int n, int kb, long routes, long experts) {
+  if (!bs && kind != KIND_W4A16) return false;
+  const long run_rows = bs ? 128 : 64;
+  const long wg = (routes / run_rows + (routes < experts ? routes : experts)) * (n / 64);
+  if (!bs) {
+    if (kb % 512 != 0 || (gs && routes < 4 * experts)) return false;
+    const bool short_k = kb <= 8192;   // model_dim of up to 4096
+    return tile_m == 64 || routes >= 24 * experts || !short_k || wg <= 512;
+  }
+  if (wg > 256 && routes >= 512 * experts) return true;
+  switch (tile_m) {
+    case 16: return wg > 384 && routes >= 32 * experts;
+    case 32:
+      return (wg > 384 && routes >= 64 * experts) || (wg >= 896 && routes >= 48 * experts) ||
+             (wg >= 1536 && routes >= 24 * experts);
+    default:
+      return (wg > 384 && routes >= 96 * experts) ||
+             (wg >= 896 && routes >= (kb > 6144 ? 4 : kb >= 4096 ? 16 : 40) * experts);
+  }
 }
 
 // Stage 2 of routings between decode and the 256-row runs of large experts: runs of 64 rows (32) on
@@ -300,7 +331,7 @@ int moe_choose(int stage, int tokens, int N, int K, int experts, int topk, int t
                          &c->tile_n, wgroup))
     return rc;
   if (stage == 1) {
-    if (moe_stage1_streams(kind, bs, wgroup, tile_m, (int)kb, routes, experts)) {
+    if (moe_stage1_streams(kind, bs, wgroup, tile_m, N, (int)kb, routes, experts)) {
       *c = MoeChoice{MoePath::kStream1, (kind == KIND_W4A16 ? 64 : 128) / tile_m, 64};
     } else if (moe_stream_stage1(stage, kind, bs) && c->r * tile_m == 128) {
       c->path = MoePath::kStream1;

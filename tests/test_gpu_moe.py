@@ -795,8 +795,8 @@ def test_single_block_wide_tiles(gpu, kind, group):
     test_w4a16_stage1_lds_tiles of test_gpu_moe_mid.py).  Stage 2 in atomic and reduce modes."""
     for tokens, s2 in ((512, (1, 64) if kind == "int4_bf16" else (2, 128)), (160, (1, 128))):
         w = W.moe_custom(tokens, 512, 1024, 64, 4, 32, 256, 256, kind, seed=11 + tokens)
-        # the stream kernel's 64- and 128-row runs of 64 columns
-        assert _chosen_tile(1, w, kind) == ((2, 64) if kind == "int4_bf16" else (4, 64))
+        # the stream kernel's 64- and 128-row runs of 64 columns (W4A16 with few routes: single blocks)
+        assert _chosen_tile(1, w, kind) == ((4, 64) if kind != "int4_bf16" else (2, 64) if tokens == 512 else (1, 64))
         assert _chosen_tile(2, w, kind) == s2
         p = W.moe_problem(w, gpu, group_size=group)
         p["group_size"] = group
@@ -824,10 +824,10 @@ def test_single_block_wide_tiles(gpu, kind, group):
 
 
 def test_single_block_wide_tiles_blockscale(gpu):
-    """The same routings through the blockscale MoE: 512 tokens -> stage 1 on the stream kernel,
-    stage 2 on 64-column tiles; 320 and 160 tokens -> stage 1 on single-block tiles of 128 and 64
-    columns, stage 2 on 64 and 128."""
-    for tokens, s1, s2 in ((512, (4, 64), (1, 64)), (320, (1, 128), (1, 64)), (160, (1, 64), (1, 128))):
+    """The same routings through the blockscale MoE: 512 tokens -> stage 1 single-block
+    128-column tiles, stage 2 64-column ones; 160 tokens -> 64 and 128 columns; 768 tokens -> stage 1
+    on the stream kernel, stage 2 on runs of 64 rows."""
+    for tokens, s1, s2 in ((512, (1, 128), (1, 64)), (160, (1, 64), (1, 128)), (768, (4, 64), (2, 128))):
         _wide_blockscale(gpu, tokens, s1, s2)
 
 

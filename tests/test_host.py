@@ -496,7 +496,22 @@ def test_moe_tile_choice_pinned():
     assert sel(1, 512, 1024, 64, 4, 32, 256, "int4_bf16", k=7232) == (1, 128)     # 128 runs x 8
     assert sel(1, 512, 1024, 64, 4, 32, 256, "int4_bf16") == (2, 64)
     assert sel(1, 320, 1024, 64, 4, 32, 128, "fp8", 1) == (1, 128)
-    assert sel(1, 512, 1024, 64, 4, 32, 128, "fp8", 1) == (4, 64)
+    assert sel(1, 512, 1024, 64, 4, 32, 128, "fp8", 1) == (1, 128)
+    assert sel(1, 768, 1024, 64, 4, 32, 128, "fp8", 1) == (4, 64)     # 48 routes per expert
+    # the stream kernel's workgroups have to fill the chip: 36 to 288 of them on 8 experts of inter_dim 256
+    for tokens, tiles in ((96, [1, 1, 1]), (1536, [1, 1, 1]), (4096, [8, 4, 2])):
+        assert [sel(1, tokens, 256, 8, 2, tm, 128, "fp8", 1, k=1024)[0] for tm in (16, 32, 64)] == tiles, tokens
+    # 16 and 32 routes per expert: 64-row blocks on whole chips only, 16-row blocks from 32
+    assert [sel(1, t, 256, 256, 8, 64, 128, "fp8", 1)[0] for t in (127, 128, 1024)] == [1, 2, 2]      # model_dim 7168
+    assert [sel(1, t, 1536, 64, 8, 64, 128, "fp8", 1, k=4096)[0] for t in (64, 127, 128)] == [1, 1, 2]
+    assert [sel(1, t, 768, 128, 8, 64, 128, "fp8", 1, k=2048)[0] for t in (256, 639, 640)] == [1, 1, 2]
+    assert [sel(1, t, 256, 256, 8, 16, 128, "fp8", 1)[0] for t in (1023, 1024)] == [1, 8]
+    assert [sel(1, t, 256, 128, 8, 32, 128, "fp8", 1)[0] for t in (512, 768, 1024)] == [1, 1, 4]      # under 896 workgroups
+    # W4A16: not for short model_dims with few routes and more than one round of workgroups
+    assert sel(1, 64, 768, 128, 8, 16, 128, "int4_bf16", k=2048)[0] == 1
+    assert sel(1, 64, 768, 128, 8, 16, 128, "int4_bf16", k=4352) == (4, 64)
+    assert sel(1, 384, 768, 128, 8, 16, 128, "int4_bf16", k=2048) == (4, 64)    # 24 routes per expert
+    assert sel(1, 4, 768, 8, 2, 16, 128, "int4_bf16", k=2048) == (4, 64)        # 96 workgroups
     assert sel(1, 160, 1024, 64, 4, 32, 256, "fp8", 1) == (1, 64)
     for kind in ("fp8", "int8", "bf16", "fp16", "int4", "int8smooth", "int4_bf16"):
         assert sel(2, 160, 512, 64, 4, 32, 256, kind) == (1, 128), kind
