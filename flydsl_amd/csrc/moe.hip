@@ -273,44 +273,100 @@ bool moe_stage1_streams(int kind, bool bs, bool gs, int tile_m, int n, int kb, l
   }
 }
 
-// Stage 2 of routings between decode and the 256-row runs of large experts: runs of 64 rows (32) on
-// the 4-wave tiles, where moe_tiles takes 256-row runs of 16-row blocks from 32 routes per expert,
-// most of them empty, or single blocks that each re-read their expert's weights.  r: moe_tiles' run.
-// Graph-timed on MI355X (us; moe_tiles' choice against 64 rows x 128 columns unless said):
-//   * 16-row blocks, inter_dim of less than 1024 bytes, atomics: from 64 routes per expert (7168 x 256:
-//     94 routes 577 against 326, 250: 500 against 389, 512: 880 against 760; bf16 250: 576 against 438);
-//     from 32, 32 rows x 64 columns (40 routes 478 against about 155; 188 with 64 rows).
-//   * deeper inter_dims (at least 1024 bytes).  16-row blocks from 32 routes per expert (4096 x 1536
-//     int8, 37 / 75 / 187 routes: atomics 173 / 236 / 255 against 90 / 114 / 198, rows 150 / 192 / 210
-//     against 108 / 132 / 221; 4096 x 14336 fp8, 37 / 75 / 175: 168 / 329 / 342 against 110 / 142 / 268).
-//     32-row blocks, atomics, the same (95 / 129 / 277 against 90 / 112 / 190; 167 / 170 / 297 against 110 /
-//     142 / 246; int4 6144 x 1024 at 62 routes 173 against 141); rows: single blocks of 128 columns
-//     (never 64: 4096 x 14336 at 37 routes 166 against 108) and 64-row runs from 128 routes (187 routes
-//     247 against 196, 175: 320 against 245; below that level or slower, as for int4: 135 against 161).
-//     64-row blocks, atomics: 128 columns in place of 64 from 48 routes (75 routes 118 against 113
-//     and 183 against 110, 187: 206 against 179; at 19 routes 78 against 90).
-//   * W4A16 and blockscale (single blocks in moe_tiles) from 48 routes: blockscale 4096 x 1536 at 125
-//     routes, 16- / 32-row blocks 288 / 250 against 183 / 181, W4A16 4096 x 14336 at 75 routes, 16-row
-//     blocks 351 against 210; at 31 routes and fewer slower.
-void moe_stage2_mid(int kind, bool bs, bool rows, int tile_m, int r, int kb, int n, long routes, long experts,
-                    int* r_out, int* tn_out) {
-  if (n % 128 != 0) return;
-  // moe_tiles' 256-row runs of large experts stay; 16-row blocks have runs from 32 routes per expert
-  const bool runs16 = !bs && kind != KIND_W4A16 && tile_m == 16;
-  const int inter = moe_a_16bit(kind) ? kb / 2 : kb;
-  if (r > 1 && !(runs16 && !moe_large_experts(kind, inter, routes, experts))) return;
-  const bool deep = kb >= 1024;
-  const long from = bs || kind == KIND_W4A16 ? 48 : 32;
-  if (routes < from * experts || (!deep && !(runs16 && !rows))) return;
-  if (tile_m == 64 && (rows || routes < 48 * experts)) return;
-  const bool narrow = !deep && routes < 64 * experts;
-  *tn_out = narrow ? 64 : 128;
-  if (tile_m == 16)
-    *r_out = narrow ? 2 : 4;
-  else if (tile_m == 32)
-    *r_out = !rows || (routes >= 128 * experts && kind != KIND_INT4) ? 2 : 1;
-  else
-    *r_out = 1;
+// Stage 2 of routings between decode and the 256-row runs of large experts: runs of 64 rows (32) and
+// 128 columns on the 4-wave tiles, where moe_tiles takes 256-row runs of 16-row blocks from 32 routes
+// per expert, most of them empty, or single blocks that each re-read their expert's weights.  *r and
+// *tn: moe_tiles' choice, replaced where this one is faster.  Graph-timed on MI355X over ten sets of
+// dims (model_dim x inter_dim, experts below), 32 to 1536 routes per expert, all kinds; us, moe_tiles'
+// choice against this one, fp8 and 64 rows x 128 columns unless said.  "Deep": inter_dim of at
+// least 1024 bytes.
+//   16-row blocks in place of 256-row runs:
+//   * shallow, atomics: 32 rows x 64 columns below 64 routes per expert (7168 x 256, 128 experts, 40
+//     routes 478 against 155), then 64 rows, at every number of routes (64 / 128 / 512 / 1536 routes
+//     2.2 / 1.5 / 1.15 / 1.06 times as fast; level at worst).
+//   * deep: while the 256-row runs are far from full, longer with atomics and for int4.  Atomics: 4096 x
+//     1536, 64 experts, 37 / 75 / 187 routes 173 / 236 / 255 against 90 / 114 / 198; up to 384 routes
+//     (6144 x 1024, 128 experts 1.01 times; 4096 x 2048, 17 experts, 512 routes 0.94); 16-bit from inter_dim
+//     1024 up to 128 (6144 x 1024 bf16, 96 / 128 / 192 / 384 routes 1.25 / 1.01 / 0.91 / 0.74), below up to 768
+//     (2048 x 768 bf16, 768 / 1536 routes 1.03 / 0.93); int4 throughout (1536 routes 1.13).  Per-route rows
+//     up to 128 (6144 x 1024, 128 / 192 routes 1.08 / 0.91), 16-bit from inter_dim 1024 up to 96, int4 up
+//     to 256 (6144 x 1024, 256 / 384 routes 1.02 / 0.90; 4096 x 1536, 512 / 1024 routes 0.91 / 0.44).
+//   * inter_dims of 4096 or more: below 64 routes, and up to 128 where the 256-row runs make fewer than
+//     256 workgroups (4096 x 14336, 8 experts, 64 / 128 / 192 routes 1.28 / 2.0 / 0.68; 8192 x 8192, 16
+//     experts, 40 / 64 / 192 routes 1.10 / 0.96 / 0.66); int4 up to 192 (1.50 / 1.10; 256 routes 0.76).
+//   16-row blocks in place of single blocks:
+//   * W4A16 and blockscale, deep, from 48 routes per expert (blockscale 4096 x 1536 at 96 routes 1.42; W4A16
+//     4096 x 14336 at 64 routes 1.53); W4A16 atomics with inter_dims of up to 512 from 96 (4096 x 512, 32
+//     experts, 48 / 96 routes 0.86 / 1.14), rows in place of 128 columns up to 64K routes (2048 x 768,
+//     128 experts, 384 / 1024 routes 1.65 / 0.94).
+//   * the other kinds (a caller's 64 columns, or a model_dim that is no multiple of 256): from 40 routes
+//     for inter_dims of at least 1024, else from 96 (4096 x 512, 64 / 96 routes 0.86 / 1.04), and not for
+//     experts of less than 1M weights, which stay in L2 (1024 x 256, 8 experts, 64 / 1536 routes
+//     5.3 / 29.9 against 7.6 / 36.3).
+//   32-row blocks, deep, in place of single blocks:
+//   * atomics (64 columns in moe_tiles) from 40 routes per expert (48 for W4A16 and blockscale) where there
+//     are 4096 routes (4096 x 1536 at 64 / 192 routes 1.08 / 1.36; 4096 x 2048, 17 experts, 64 routes 0.90,
+//     256 routes 1.40) or inter_dim is at least 4096 (4096 x 14336 at 32 / 40 / 64 routes 0.88 / 1.45 / 1.21).
+//   * rows: from 128 routes (4096 x 1536 at 128 / 256 routes 1.16 / 1.48); W4A16 in place of 128 columns
+//     while there are fewer than 48K (2048 x 768, 128 experts, 256 / 768 routes 1.14 / 0.92).  128-column
+//     single blocks in place of moe_tiles' 64 for int4, blockscale and W4A16 below that (int4 with a
+//     caller's 64 columns 1.3-1.6), for the other kinds where moe_tiles' decode rule (512 routes) takes 64
+//     columns for few large experts (4096 x 14336, 8 experts, 40 / 64 routes 1.53 / 1.23; 8192 x 8192,
+//     16 experts, 64 routes in place of a caller's 64 columns 0.86).
+//   64-row blocks, deep, atomics: 128 columns in place of 64, from 48 routes per expert for blockscale
+//   (1.2-1.3; 4096 x 14336 at 96 routes 2.07); else from 4096 routes for inter_dims of at least 768, 1024 for
+//   group scales (6144 x 1024 1.04-1.12, 4096 x 1536 1.03-1.15; 4096 x 2048, 17 experts, 64 to 192 routes
+//   0.86-0.96; 4096 x 512 bf16 0.86-0.99), and not for int4 and per-row W4A16 (0.83-1.06).  inter_dims of 4096
+//   or more: 96 to 128 routes (4096 x 14336, 64 / 96 / 128 / 192 routes 0.96 / 1.61 / 1.31 / 0.88), int4 and
+//   group scales on (int4 at 192 routes 1.29, 8192 x 8192 at 384 routes 1.31).
+void moe_stage2_mid(int kind, bool bs, bool gs, bool rows, int tile_m, int n, int k, long routes, long experts, int* r,
+                    int* tn) {
+  const bool w4 = kind == KIND_W4A16, i4 = kind == KIND_INT4, two = moe_a_16bit(kind);
+  const bool deep = (two ? 2 : 1) * k >= 1024;
+  // moe_tiles' 256-row runs of large experts stay; 16-row blocks of these kinds have runs from 32 routes
+  const bool runs16 = !bs && !w4 && tile_m == 16;
+  if (n % 128 != 0 || (*r > 1 && !(runs16 && !moe_large_experts(kind, k, routes, experts)))) return;
+  auto from = [&](long per_expert) { return routes >= per_expert * experts; };
+  auto upto = [&](long per_expert) { return routes <= per_expert * experts; };
+  if (!from(bs || w4 ? 48 : 32) || (!deep && !(runs16 && !rows))) return;
+  bool take;
+  if (tile_m == 16) {
+    if (bs)
+      take = true;
+    else if (w4)
+      take = rows ? *tn == 64 || routes < 65536 : k > 512 || from(96);
+    else if (*r == 1)
+      take = (long)n * k >= 1 << 20 && from(k >= 1024 ? 40 : 96);
+    else if (!deep)
+      take = true;
+    else if (k >= 4096)
+      take = i4 ? upto(192)
+                : !from(64) || (upto(128) && (routes / 256 + (routes < experts ? routes : experts)) * (n / 256) < 256);
+    else if (rows)
+      take = upto(i4 ? 256 : two && k >= 1024 ? 96 : 128);
+    else
+      take = i4 || upto(!two ? 384 : k >= 1024 ? 128 : 768);
+    if (!take) return;
+    const bool narrow = !deep && !from(64);
+    *r = narrow ? 2 : 4;
+    *tn = narrow ? 64 : 128;
+  } else if (tile_m == 32) {
+    if (!rows)
+      take = from(40) && (k >= 4096 || routes >= 4096);
+    else if (w4)
+      take = *tn == 64 || routes < 49152;
+    else
+      take = bs || i4 || from(128) || (from(40) && routes <= 512);
+    if (!take) return;
+    *r = !rows || (from(128) && !i4) ? 2 : 1;
+    *tn = 128;
+  } else {
+    if (rows || !from(48)) return;
+    take = bs || (k >= 4096 && from(96) && (i4 || upto(128))) ||
+           (!i4 && (!w4 || gs) && routes >= 4096 && k >= (gs ? 1024 : 768) && (k < 4096 || gs));
+    if (!take) return;
+    *tn = 128;
+  }
 }
 
 // What a call runs: a kernel family, R routing blocks per run and tile_n output columns.
@@ -367,7 +423,7 @@ int moe_choose(int stage, int tokens, int N, int K, int experts, int topk, int t
       return 0;
     }
   }
-  moe_stage2_mid(kind, bs, rows, tile_m, c->r, (int)kb, N, routes, experts, &c->r, &c->tile_n);
+  moe_stage2_mid(kind, bs, wgroup, rows, tile_m, N, K, routes, experts, &c->r, &c->tile_n);
   return 0;
 }
 

@@ -790,10 +790,10 @@ WIDE_KINDS = [("fp8", -1), ("int8", -1), ("bf16", -1), ("fp16", -1), ("int4", -1
 def test_single_block_wide_tiles(gpu, kind, group):
     """Routings with about one block per expert (top-4 of 64 experts, D = 512, I = 1024, tile_m
     32, tile_n hints 256), checked through flygemm_moe_select_tile first: 512 tokens -> stage 2 with
-    atomics on runs of 64 rows (W4A16: 64-column tiles; 32 routes per expert), 160 tokens -> on the 128-column kernel (10
+    atomics on 64-column tiles (32 routes per expert), 160 tokens -> on the 128-column kernel (10
     routes per expert).  Stage 1 runs the stream kernel (W4A16 on its LDS-staged tiles:
     test_w4a16_stage1_lds_tiles of test_gpu_moe_mid.py).  Stage 2 in atomic and reduce modes."""
-    for tokens, s2 in ((512, (1, 64) if kind == "int4_bf16" else (2, 128)), (160, (1, 128))):
+    for tokens, s2 in ((512, (1, 64)), (160, (1, 128))):
         w = W.moe_custom(tokens, 512, 1024, 64, 4, 32, 256, 256, kind, seed=11 + tokens)
         # the stream kernel's 64- and 128-row runs of 64 columns (W4A16 with few routes: single blocks)
         assert _chosen_tile(1, w, kind) == ((4, 64) if kind != "int4_bf16" else (2, 64) if tokens == 512 else (1, 64))
@@ -826,8 +826,8 @@ def test_single_block_wide_tiles(gpu, kind, group):
 def test_single_block_wide_tiles_blockscale(gpu):
     """The same routings through the blockscale MoE: 512 tokens -> stage 1 single-block
     128-column tiles, stage 2 64-column ones; 160 tokens -> 64 and 128 columns; 768 tokens -> stage 1
-    on the stream kernel, stage 2 on runs of 64 rows."""
-    for tokens, s1, s2 in ((512, (1, 128), (1, 64)), (160, (1, 64), (1, 128)), (768, (4, 64), (2, 128))):
+    on the stream kernel, stage 2 as with 512."""
+    for tokens, s1, s2 in ((512, (1, 128), (1, 64)), (160, (1, 64), (1, 128)), (768, (4, 64), (1, 64))):
         _wide_blockscale(gpu, tokens, s1, s2)
 
 

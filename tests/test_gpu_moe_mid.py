@@ -53,11 +53,11 @@ def test_blockscale_stage1_stream(gpu, tile_m, tokens):
         M._check(out, M.ref_bs1(p, K % 256 == 0, rows), rows, what=f"blockscale tm{tile_m} t{tokens} K{K}")
 
 
-def _reduce(p, gpu, kind, out_dtype):
+def _reduce(p, gpu, kind, out_dtype, group=-1):
     w = p["workload"]
     fn = compile_moe_gemm2_ex(model_dim=w.model_dim, inter_dim=w.inter_dim, experts=w.experts, topk=w.topk,
                               tile_m=w.tile_m, tile_n=w.tile_n2, tile_k=M._tile_k(kind), doweight_stage2=True, in_dtype=kind,
-                              out_dtype=out_dtype, mode=MoeGemm2Mode.REDUCE)
+                              out_dtype=out_dtype, mode=MoeGemm2Mode.REDUCE, group_size=group)
     out = torch.full((w.tokens, w.model_dim), float("nan"), dtype=M.OUT_T[out_dtype], device=gpu)
     empty = torch.empty(0, dtype=torch.float32, device=gpu)
     fn(out, H.dev_flat(p["a2"], gpu), H.dev_flat(p["w2_shuf"], gpu), empty if p["sa2"] is None else p["sa2"],
@@ -66,7 +66,7 @@ def _reduce(p, gpu, kind, out_dtype):
     return out
 
 
-# kind, inter_dim, tokens (top-2 of 5 experts: 40, 60 and 160 routes per expert)
+# kind, inter_dim, tokens (top-2 of 5 experts: 40, 60 and 160 routes per expert), on whatever tile they take
 STAGE2 = [("fp8", 256, 100), ("fp8", 256, 400), ("bf16", 128, 100), ("bf16", 256, 400), ("int4", 256, 100), ("fp8", 1024, 100),
           ("fp8", 1152, 400), ("int8", 1024, 150), ("int4", 1024, 400), ("fp16", 512, 150), ("bf16", 576, 400),
           ("int4_bf16", 512, 150), ("int4_bf16", 1024, 400)]
@@ -84,6 +84,43 @@ def test_stage2_mid(gpu, kind, inter, tokens, tile_m, model_dim):
         M.check_stage2(p, out, True, what=f"{what} atomics {out_dtype}",
                        atol_rms=M.BF16_ATOMIC_ATOL if out_dtype == "bf16" else 1e-2)
     M.check_stage2(p, _reduce(p, gpu, kind, "bf16"), True, what=f"{what} rows", route_round="bf16")
+
+
+# The tiles of the routings in between, each reached on purpose: kind, group, tokens, model_dim, inter_dim, experts,
+# top-k, tile_m, tile_n, tile with atomics (None: the query does not cover group scales)
+TILES = [("fp8", -1, 100, 256, 256, 5, 2, 16, 128, (2, 64)), ("int4", -1, 100, 256, 256, 5, 2, 16, 128, (2, 64)),
+         ("fp8", -1, 400, 256, 256, 5, 2, 16, 128, (4, 128)), ("bf16", -1, 150, 256, 512, 5, 2, 16, 128, (4, 128)),
+         ("int8", -1, 400, 256, 1024, 5, 2, 16, 128, (4, 128)), ("int4", -1, 400, 256, 1024, 5, 2, 16, 128, (4, 128)),
+         ("fp16", -1, 300, 256, 1024, 5, 2, 16, 128, (4, 128)), ("bf16", -1, 400, 256, 1024, 5, 2, 16, 128, (16, 256)),
+         ("fp8", -1, 100, 256, 4096, 5, 2, 16, 128, (4, 128)), ("fp8", -1, 180, 1152, 1024, 5, 2, 16, 128, (4, 128)),
+         ("int4_bf16", -1, 150, 256, 1024, 5, 2, 16, 128, (4, 128)), ("int4_bf16", -1, 500, 384, 512, 5, 2, 16, 128, (4, 128)),
+         ("fp8", -1, 100, 256, 4096, 5, 2, 32, 128, (2, 128)), ("int4", -1, 100, 384, 4096, 5, 2, 32, 128, (2, 128)),
+         ("bf16", -1, 1100, 256, 1024, 12, 4, 32, 128, (2, 128)), ("int4_bf16", -1, 150, 256, 4096, 5, 2, 32, 128, (2, 128)),
+         ("fp8", -1, 280, 256, 4096, 5, 2, 64, 128, (1, 128)), ("int8", -1, 1100, 256, 1024, 12, 4, 64, 128, (1, 128)),
+         # group scales at 60 and 200 routes per expert
+         ("int4_bf16", 32, 150, 256, 512, 5, 2, 16, 128, None), ("int4_bf16", 32, 500, 256, 1024, 5, 2, 16, 128, None),
+         ("int4_bf16", 32, 150, 256, 4096, 5, 2, 32, 128, None), ("int4_bf16", 32, 1200, 256, 512, 12, 4, 32, 128, None),
+         ("int4_bf16", 32, 150, 256, 1024, 5, 2, 64, 128, None), ("int4_bf16", 32, 600, 384, 1024, 12, 4, 64, 128, None),
+         ("int4_bf16", 32, 1100, 256, 1024, 12, 4, 64, 128, None)]
+
+
+@pytest.mark.parametrize("case", TILES, ids=lambda c: "-".join(str(v) for v in c[:9]))
+def test_stage2_mid_tiles(gpu, case):
+    kind, group, tokens, model_dim, inter, experts, topk, tile_m, tile_n, tile = case
+    w = W.moe_custom(tokens, model_dim, inter, experts, topk, tile_m, 64, tile_n, kind, seed=inter + tokens + tile_m)
+    if tile is not None:
+        assert M._chosen_tile(2, w, kind) == tile
+    p = W.moe_problem(w, gpu, group_size=group)
+    p["group_size"] = group
+    rows = np.unique(np.r_[np.arange(0, tokens, 7), tokens - 1])
+    for out_dtype in ("f16", "f32", "bf16"):
+        out = M.run_stage2(p, gpu, out_dtype, doweight=True)
+        assert torch.isfinite(out.float()).all()
+        M.check_stage2(p, out, True, rows, rows, what=f"{case} atomics {out_dtype}",
+                       atol_rms=M.BF16_ATOMIC_ATOL if out_dtype == "bf16" else 1e-2)
+    out = _reduce(p, gpu, kind, "bf16", group)
+    assert torch.isfinite(out.float()).all()
+    M.check_stage2(p, out, True, rows, rows, what=f"{case} rows", route_round="bf16")
 
 
 @pytest.mark.parametrize("tile_m", [16, 32, 64])

@@ -486,6 +486,25 @@ def test_moe_tile_choice_pinned():
     assert sel(2, 160, 7168, 128, 8, 64, 256) == (1, 128)     # 10 routes per expert
     assert sel(2, 8192, 7168, 128, 8, 16, 256) == (4, 128)
     assert sel(2, 8192, 7168, 128, 8, 16, 256, "int4") == (4, 128)
+    # between decode and large experts: runs of 64 rows while 256-row runs are far from full (longer for
+    # int4), and where single blocks re-read their weights, unless those stay in L2
+    assert [sel(2, t, 7168, 128, 8, 16, 256) for t in (512, 1024)] == [(2, 64), (4, 128)]     # 32 and 64 routes per expert
+    for tokens, tile in ((512, (4, 128)), (3072, (4, 128)), (3073, (16, 256))):     # 64, 384 and more per expert
+        assert sel(2, tokens, 4096, 64, 8, 16, 256, k=1536) == tile
+        assert sel(2, tokens, 4096, 64, 8, 16, 256, "int4", k=1536) == (4, 128)
+    assert [sel(2, t, 4096, 64, 8, 16, 256, "bf16", k=1536)[0] for t in (1024, 1025)] == [4, 16]      # 128
+    assert [sel(2, t, 2048, 128, 8, 16, 256, "bf16", k=768)[0] for t in (12288, 12289)] == [4, 16]    # 768
+    assert [sel(2, t, 4096, 8, 2, 16, 256, k=14336)[0] for t in (512, 513)] == [4, 16]                # 128
+    assert [sel(2, t, 8192, 16, 4, 16, 256, k=8192)[0] for t in (255, 256)] == [4, 16]                # 64
+    assert [sel(2, t, 8192, 16, 4, 16, 256, "int4", k=8192)[0] for t in (768, 769)] == [4, 16]        # 192
+    assert [sel(2, t, 4096, 32, 4, 16, 64)[0] for t in (383, 767, 768)] == [1, 1, 4]                  # a caller's 64 columns
+    assert sel(2, 4096, 1024, 8, 2, 16, 64) == (1, 64)                              # experts of 256K weights
+    assert [sel(2, t, 4096, 64, 8, 32, 256, k=1536) for t in (511, 512)] == [(1, 64), (2, 128)]       # 4096 routes
+    assert [sel(2, t, 4096, 8, 2, 32, 256, k=14336) for t in (159, 160)] == [(1, 64), (2, 128)]       # 40 per expert
+    assert [sel(2, t, 4096, 64, 8, 64, 256, k=1536) for t in (511, 512)] == [(1, 64), (1, 128)]
+    assert sel(2, 2048, 4096, 64, 8, 64, 256, "int4", k=1536) == (1, 64)
+    assert [sel(2, t, 4096, 8, 2, 64, 256, k=14336)[1] for t in (383, 384, 512, 513)] == [64, 128, 128, 64]
+    assert [sel(2, t, 4096, 32, 4, 16, 256, "int4_bf16", k=512)[0] for t in (767, 768)] == [1, 4]     # 96 per expert
     # decode: 64-column single-block tiles whatever the caller asked
     assert sel(1, 8, 256, 256, 8, 32, 256, "int4_bf16", k=7232) == (1, 64)
     assert sel(1, 8, 256, 256, 8, 32, 256, "int4_bf16") == (2, 64)      # whole 256-element steps: 64-row runs
