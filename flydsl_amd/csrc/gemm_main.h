@@ -155,12 +155,28 @@ __device__ __forceinline__ void workgroup_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Instructions in front of a kernel's code that shift its main loop within the 32-byte windows in
+// which instructions are fetched.  Graph-timed on MI355X over 16 placements of the same code, 4 bytes
+// apart: int8 256 x 256 tiles take 51.4 to 51.9 us for 4096 x 4096 x 4096 (fastest with the loop's first
+// instruction at byte 0 or 4 of a window) and int4 64 x 128 tiles 19.1 to 19.3 us for 256 x 14336 x 4096
+// (at byte 16 to 24), both with period 32; fp8 and bf16 256 x 256 tiles stay within the runs' spread.
+// The numbers go with the prologues that the compiler makes of this file:
+// tests/test_code_placement.py checks where the loops lie.
+template <int BM, int BN, int WM, int KIND, int EPI, int KSUB>
+__device__ __forceinline__ void place_main_loop() {
+  if constexpr (KIND == KIND_INT8 && BM == 256 && BN == 256 && WM == 2 && EPI == EPI_ROWCOL)
+    asm volatile(".rept 4\n\ts_nop 0\n\t.endr");
+  else if constexpr (KIND == KIND_INT4 && BM == 64 && BN == 128 && KSUB == 1 && EPI == EPI_ROWCOL)
+    asm volatile(".rept 5\n\ts_nop 0\n\t.endr");
+}
+
 // KSUB: K tiles per pipeline step (two-stage ring only).  With 2, each LDS stage holds two
 // 128-byte K tiles and a step waits for, and multiplies, both: half the barriers and twice the
 // bytes in flight per wait, for tiles whose steps are short next to the DMA latency.
 template <int BM, int BN, int WM, int WN, int KIND, int EPI, bool OUT_BF16, int KSUB = 1>
 __global__ void __launch_bounds__(WM * WN * 64, 1) gemm_main_kernel(GemmArgs p) {
   using C = MainCfg<BM, BN, WM, WN, KIND>;
+  place_main_loop<BM, BN, WM, KIND, EPI, KSUB>();
   static_assert(KSUB == 1 || (KSUB == 2 && C::NS == 2 && EPI != EPI_BLOCK && KIND != KIND_FP4),
                 "two K tiles per step: two-stage ring, no per-K-tile scales");
   constexpr int MR = C::MR, NR = C::NR, NW = C::NW;
