@@ -537,7 +537,7 @@ QuantLaunch quant_fn(int M, int N) {
                                 : quant_rows_kernel<IN, OUT, MODE, 0, NT>;
     return QuantLaunch{fn, 1, NT};
   };
-  if (N >= kQuantWideN || M <= kQuantFewRows) return pick(std::integral_constant<int, 512>{});
+  if (N >= kQuantWideN || (M <= kQuantFewRows && N > 256 * 8)) return pick(std::integral_constant<int, 512>{});
   return pick(std::integral_constant<int, 256>{});
 }
 

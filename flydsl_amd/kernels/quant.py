@@ -46,8 +46,9 @@ def build_quant_module(N: int):
     N = int(N)
     if N <= 0 or N % VEC_WIDTH:
         raise ValueError(f"N={N} must be a positive multiple of {VEC_WIDTH}")
-    # the library runs rows of WIDE_N or more elements with twice the threads (kQuantWideN in
-    # csrc/quant_rows.h): each thread still owns VEC_WIDTH consecutive elements per slice
+    # the reference's configuration keys, from N alone (twice the threads from WIDE_N elements).  They
+    # are nominal: the library also chooses by the number of rows, with several rows per workgroup
+    # for short ones (csrc/quant_rows.h)
     threads = 2 * BLOCK_THREADS if N >= WIDE_N else BLOCK_THREADS
     tile_cols = threads * VEC_WIDTH
 

@@ -50,15 +50,21 @@ def test_rows(gpu, dtype, qd, rounding):
 
 
 def test_reference_kernel_form(gpu):
+    """Every kernel of the dispatch in this form too.  Nothing is scrubbed: NaN is left out of the row's
+    maximum and gives code 0, infinity gives scale infinity and codes 0."""
     for N in EDGES:
-        x = _rows(N, torch.float16, N)[:6]
-        q_ref, s_ref = oq.quant_rows_recip(x.numpy())
-        launch, _ = build_quant_module(N)
-        q = torch.empty(6, N, dtype=torch.int8, device=gpu)
-        s = torch.empty(6, dtype=torch.float32, device=gpu)
-        launch(x.to(gpu), q, s, 6)
-        assert np.array_equal(s.cpu().numpy().view(np.uint32), s_ref.reshape(-1).view(np.uint32))
-        assert np.array_equal(q.cpu().numpy(), q_ref)
+        x = _rows(N, torch.float16, N)
+        q_ref, s_ref = oq.quant_rows_recip(torch.nan_to_num(x, nan=0.0, posinf=0.0, neginf=0.0).numpy())
+        q_ref[[6, 8]], s_ref[[6, 8]] = 0, np.inf
+        for copies, extra in ((1, 0), (36, 3), (142, 1)):   # 29, 1047 and 4119 rows
+            xb = torch.cat([x.repeat(copies, 1), x[:extra]]).to(gpu)
+            rows = np.arange(xb.shape[0]) % 29
+            launch, _ = build_quant_module(N)
+            q = torch.empty(xb.shape[0], N, dtype=torch.int8, device=gpu)
+            s = torch.empty(xb.shape[0], dtype=torch.float32, device=gpu)
+            launch(xb, q, s, xb.shape[0])
+            assert np.array_equal(s.cpu().numpy().view(np.uint32), s_ref.reshape(-1).view(np.uint32)[rows]), (N, copies)
+            assert np.array_equal(q.cpu().numpy(), q_ref[rows]), (N, copies)
 
 
 def test_quotients_are_the_divisions(gpu):
