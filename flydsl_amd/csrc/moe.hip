@@ -158,10 +158,10 @@ int moe_tiles(int stage, int tokens, int N, int K, int experts, int topk, int ti
       return 0;
     }
   }
-  // Stage 1 of 1-byte, 16-bit and W4A8 weights: the stream kernel, 128-row runs of 64 columns
-  // (every N here is a multiple of 64: tile_n, checked by the callers, divides it).  The
+  // Stage 1 of 1-byte, 16-bit and W4A8 weights: the stream kernel, 128-row runs of 64 columns.  The
   // caller's tile_n is a hint throughout: tiling does not change results.
   if (moe_stream_stage1(stage, kind, bs)) {
+    if (N % 64 != 0) return fail(hipErrorInvalidValue, "%s: N=%d must be a multiple of tile_n=64", what, N);
     *r_out = 128 / tile_m;
     *tn_out = 64;
     return 0;

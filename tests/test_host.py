@@ -590,6 +590,17 @@ def test_moe_tile_choice_pinned():
     assert sel(1, 16, 256, 4, 2, 16, 64, "fp4") != 0 and b"in_dtype" in lib.flygemm_last_error()
 
 
+def test_moe_inter_dim_of_no_whole_column_tile_is_refused():
+    """With tile_n = 0 (the library's choice) too: the 64-column tiles would leave columns out."""
+    import ctypes
+    lib = _lib.load()
+    p = ctypes.c_void_p(256)
+    for kind in ("fp8", "int8", "int4", "bf16", "int4_bf16"):
+        for n in (80, 32, 320 + 16):
+            rc = lib.flygemm_moe_gemm1(p, p, p, p, p, p, p, p, p, 16, n, 512, 6, 4, 2, 16, 0, _lib.FLYGEMM_IN[kind], 1, 0, -1, None)
+            assert rc != 0 and b"multiple of tile_n=64" in lib.flygemm_last_error(), (kind, n, lib.flygemm_last_error())
+
+
 def test_moe_tile_choice_reaches_built_kernels():
     """Over a spread of sizes, every choice is a tile that the kernel tables hold for its kind: a call
     with another one would be refused."""
