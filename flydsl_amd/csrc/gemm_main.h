@@ -76,8 +76,10 @@ struct MainCfg {
 // ntiles % 8 XCDs one tile more), and the grouped order walks GROUP_M tile-rows at a time so tiles in
 // flight together share A rows and B columns in that XCD's L2.  Tile counts that are no multiple of 8
 // went round-robin before, so an XCD's tiles in flight shared one panel of A and read as many panels
-// of B as tiles: bf16 5133x5120x8320 (420 tiles) 350 us against 381 on MI355X, bf16 2100x7168x4096
-// 96.7 against 100.5, fp8 5133x5120x8320 172 against 177, MXFP4 5133x8192x8192 170.8 against 173.3.
+// of B as tiles.  Graph-timed on MI355X over four sets of operands in turn, which then come from
+// HBM: bf16 5133x5120x8320 (420 tiles) 356 us against 398, bf16 2100x7168x4096 105.2 against 109.3,
+// fp8 5133x5120x8320 177 against 197, MXFP4 5133x8192x8192 level (165.7 / 164.9); with one set,
+// which the memory-side cache holds, all level.
 __device__ __forceinline__ void tile_coords(int t, int ntiles, int nbm, int& bm, int& bn) {
   const int nbn = ntiles / nbm;
   const int xcd = t & 7;

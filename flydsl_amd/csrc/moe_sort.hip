@@ -14,9 +14,10 @@
 // (a stable sort without a comparison) and no two lanes ever add to one counter at once, however
 // skewed the routing is.  Padding rows, block experts and totals are spread over all workgroups.
 //
-// Measured on MI355X, back-to-back calls of moe_sorting: 8 tokens, 256 experts, top-8 16.5 us
-// against 398 for the operators it stands in for (about 40 launches and two waits for the device);
-// 8192 tokens, 128 experts 20.0 against 439; 65536 tokens, 256 experts 25.1 against 578.
+// Measured on MI355X, top-8, graph-timed / in back-to-back calls of moe_sorting from Python: 8 tokens,
+// 256 experts 6.9 / 16.5 us against 400 for the calls of the operators it stands in for (about 40 launches and
+// two waits for the device); 8192 tokens, 128 experts 17.0 / 21 against 440-460; 65536 tokens, 256 experts
+// 25.1 / 25.1 against 578.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -33,8 +34,9 @@ static_assert(kMaxExperts <= kThreads && kMaxExperts % 64 == 0, "one thread per 
 // routes per workgroup, one launch / two
 constexpr int kChunkOne = 1024, kChunkTwo = 4096;
 // Routes up to which every workgroup counts all of them (one launch).  Graph-timed on MI355X: one
-// launch 6.6 us at 64 routes, 8.4 at 4096 and 16.9 at 16384, as much as two launches take from there
-// to 65536 routes (16.3-16.9); the extra launch also costs the host 2.5 us.
+// launch 6.9 us at 64 routes, 8.4 at 4096, 11.5 at 8192 and 16.9 at 16384, as much as two launches take
+// from 8200 routes (16.7) to 65536 (17.0, 18.5 with 256 experts); the extra launch also costs the
+// host 2.5 us.
 constexpr int kOneLaunchRoutes = 8192;
 
 struct SortArgs {

@@ -35,7 +35,8 @@
 // A DMA is inline assembly that the compiler does not track; its wait is explicit: at the top
 // of step s the only operations issued after A(s) are the weights of step s-1+Lb (LPS of them).
 // The compiler waits for a weight set counting only the later weight loads it knows of, so the
-// untracked DMAs issued after that set make it also wait for the oldest Lb*AQ operations issued
+// untracked DMAs issued after that set (KS * AQ per step, and one more in the first waves of
+// blockscale for the rows' scales) make it also wait for as many of the oldest operations issued
 // after the set: A(s) (already waited for) and some weights of step s+1, issued a step earlier.
 // The loop runs whole groups of D steps (the register set of each step is static there and
 // every path through a group issues every load); the last nk % D steps form a tail in which the

@@ -59,8 +59,8 @@ def moe_sorting(topk_ids: torch.Tensor, topk_weights: torch.Tensor, num_experts:
     M, topk = topk_ids.shape
     max_pad = M * topk + E * bs - topk
     # On the GPU: the counting-sort kernel (csrc/moe_sort.hip) in place of about 40 operators, two
-    # of which (bincount, torch.tensor) wait for the device.  Measured on MI355X, back to back: 8
-    # tokens, 256 experts, top-8 16.5 us against 398; 8192 tokens, 128 experts, top-8 20.0 against 439.
+    # of which (bincount, torch.tensor) wait for the device.  Measured on MI355X, calls back to
+    # back: 8 tokens, 256 experts, top-8 16.5 us against 400; 8192 tokens, 128 experts, top-8 21 against 440-460.
     # More experts than the kernel's counters, a top-k above the experts (whose rows may not fit
     # the buffers), empty routings and masks shorter than the experts take the operators below.
     if (0 < topk <= E <= _lib.MOE_SORT_MAX_EXPERTS and M > 0 and max_pad < 2**31 - 2**16
