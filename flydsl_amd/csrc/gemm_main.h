@@ -79,11 +79,19 @@ struct MainCfg {
 // of B as tiles.  Graph-timed on MI355X over four sets of operands in turn, which then come from
 // HBM: bf16 5133x5120x8320 (420 tiles) 356 us against 398, bf16 2100x7168x4096 105.2 against 109.3,
 // fp8 5133x5120x8320 177 against 197, MXFP4 5133x8192x8192 level (165.7 / 164.9); with one set,
-// which the memory-side cache holds, all level.
+// which the memory-side cache holds, all level; over 420 drawn shapes with such counts 1.06x.
+// FROM: with more tile rows than a group and fewer than FROM tile columns, such counts stay
+// round-robin.  There a round-robin XCD reads hardly more panels (32 tiles in flight: one of A per group
+// and nbn of B, against 8 and 4), and it gets its share of the last, partly empty tile row, which a
+// contiguous range gives to the last XCD alone: 256 x 256 tiles, fp8 6208x2448x1408 (25 x 10 tiles) 24.4 us
+// round-robin against 25.5, bf16 39.0 against 40.0, int4 (B panels of half the bytes) 6401x6336x1664 (26 x 25)
+// 84.7 against 89.6, 7763x6784x1024 (31 x 27) 0.96 times as fast.
+template <int FROM>
 __device__ __forceinline__ void tile_coords(int t, int ntiles, int nbm, int& bm, int& bn) {
   const int nbn = ntiles / nbm;
   const int xcd = t & 7;
-  t = xcd * (ntiles >> 3) + min(xcd, ntiles & 7) + (t >> 3);
+  if (FROM == 0 || (ntiles & 7) == 0 || nbm <= FLY_GROUP_M || nbn >= FROM)
+    t = xcd * (ntiles >> 3) + min(xcd, ntiles & 7) + (t >> 3);
   constexpr int GROUP_M = FLY_GROUP_M;
   const int per_group = GROUP_M * nbn;
   const int g = t / per_group;
@@ -167,7 +175,7 @@ __device__ __forceinline__ void workgroup_barrier() {
 template <int BM, int BN, int WM, int KIND, int EPI, int KSUB>
 __device__ __forceinline__ void place_main_loop() {
   if constexpr (KIND == KIND_INT8 && BM == 256 && BN == 256 && WM == 2 && EPI == EPI_ROWCOL)
-    asm volatile(".rept 4\n\ts_nop 0\n\t.endr");
+    asm volatile(".rept 2\n\ts_nop 0\n\t.endr");
   else if constexpr (KIND == KIND_INT4 && BM == 64 && BN == 128 && KSUB == 1 && EPI == EPI_ROWCOL)
     asm volatile(".rept 5\n\ts_nop 0\n\t.endr");
 }
@@ -614,7 +622,7 @@ __global__ void __launch_bounds__(WM * WN * 64, 1) gemm_main_kernel(GemmArgs p) 
   const int nitems = ntiles;
   auto item = [&](int w, int& m0_, int& n0_, int& kb_, int& ke_) {
     int bm, bn;
-    tile_coords(w, ntiles, nbm, bm, bn);
+    tile_coords<(BM == 256 && BN == 256 ? (KIND == KIND_INT4 ? 28 : 14) : 0)>(w, ntiles, nbm, bm, bn);
     m0_ = bm * BM;
     n0_ = bn * BN;
     kb_ = 0;
