@@ -634,9 +634,15 @@ int reduce_launch(void* y, const void* x, const void* mask, int tokens, int topk
   const long n = (long)tokens * (D / (dtype == FLYGEMM_OUT_F32 ? 4 : 8));
   const long g = (n + 255) / 256;
   if (g >= (1L << 31)) return fail(hipErrorInvalidValue, "moe_reduce: too large");
-  void (*fn)(void*, const void*, const int8_t*, int, int, int) =
-      dtype == FLYGEMM_OUT_FP16 ? moe_reduce_kernel<0> : dtype == FLYGEMM_OUT_BF16 ? moe_reduce_kernel<1>
-                                                                                   : moe_reduce_kernel<2>;
+  typedef void (*ReduceFn)(void*, const void*, const int8_t*, int, int, int);
+  auto pick = [&](auto dt) -> ReduceFn {
+    constexpr int DT = decltype(dt)::value;
+    if (topk >= 8) return mask ? moe_reduce_kernel<DT, true, true> : moe_reduce_kernel<DT, false, true>;
+    return mask ? moe_reduce_kernel<DT, true, false> : moe_reduce_kernel<DT, false, false>;
+  };
+  const ReduceFn fn = dtype == FLYGEMM_OUT_FP16   ? pick(std::integral_constant<int, 0>{})
+                      : dtype == FLYGEMM_OUT_BF16 ? pick(std::integral_constant<int, 1>{})
+                                                  : pick(std::integral_constant<int, 2>{});
   hipLaunchKernelGGL(fn, dim3((unsigned)g), dim3(256), 0, stream, y, x, (const int8_t*)mask, tokens, topk, D);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(e, "launch of moe_reduce failed: %s", hipGetErrorString(e));

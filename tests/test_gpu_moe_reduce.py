@@ -54,6 +54,30 @@ def test_one_call_equals_two_steps(gpu, tokens, topk, dim, tile_m, out_dtype, ke
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("topk", [1, 2, 7, 8, 9, 15, 16, 17, 25])
+def test_reduction_groups_and_remainders(gpu, dt, topk):
+    """Every form of the reduction, bit for bit: fp32 sums in slot order, one rounding, masked slots
+    not read (they hold NaN)."""
+    tokens, dim = 67, 264
+    dtype = torch.float32 if dt == "f32" else _DT[dt]
+    g = torch.Generator().manual_seed(topk)
+    x = torch.randn(tokens, topk, dim, generator=g).to(dtype)
+    mask = (torch.rand(tokens, topk, generator=g) < 0.7).to(torch.int8)
+    mask[3] = 0
+    for use_mask in (False, True):
+        want = torch.zeros(tokens, dim)
+        for s in range(topk):
+            want = torch.where((mask[:, s:s + 1] != 0) if use_mask else torch.tensor(True), want + x[:, s].float(), want)
+        xs = x.clone()
+        if use_mask:
+            xs[mask == 0] = float("nan")
+        y = torch.empty(tokens, dim, dtype=dtype, device=gpu)
+        compile_moe_reduction(topk=topk, model_dim=dim, dtype_str=dt, use_mask=use_mask)(
+            xs.to(gpu).view(-1), y.view(-1), mask.to(gpu).view(-1) if use_mask else None, tokens)
+        assert torch.equal(y.cpu(), want.to(dtype))
+
+
 def test_other_stream(gpu):
     """Called for another stream than the current one: everything runs there."""
     tokens, topk, dim = 1025, 8, 1024
