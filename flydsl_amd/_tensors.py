@@ -12,10 +12,10 @@ def plain(*ts) -> bool:
     # first of all: torch.compile can trace this question, and none of those about torch's mode stacks
     if torch.compiler.is_compiling():
         return False
-    if any(type(t) is not torch.Tensor or t.layout is not torch.strided or t.is_neg() for t in ts):
-        return False
-    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
-        return False
+    grad = torch.is_grad_enabled()
+    for t in ts:
+        if type(t) is not torch.Tensor or t.layout is not torch.strided or t.is_neg() or (grad and t.requires_grad):
+            return False
     C = torch._C
     return not (C._len_torch_dispatch_stack() or C._len_torch_function_stack() or C._get_tracing_state() is not None
                 or C._functorch.peek_interpreter_stack() is not None
@@ -25,8 +25,13 @@ def plain(*ts) -> bool:
 def plain_cuda(*ts) -> bool:
     """Tensors whose values a kernel may read and write by pointer in place of torch's own
     operators: ``plain`` ones of one GPU."""
-    dev = ts[0].device
-    return dev.type == "cuda" and all(t.device == dev for t in ts) and plain(*ts)
+    if not plain(*ts):
+        return False
+    index = ts[0].get_device()
+    for t in ts:
+        if not t.is_cuda or t.get_device() != index:
+            return False
+    return True
 
 
 def on_device(dev):
